@@ -40,7 +40,7 @@ def log(*a):
 
 
 KERNEL_NAMES = {"select": "k_select", "products": "k_products", "tridiag": "k_tridiag",
-                "ql": "k_ql_log", "apply": "k_vec", "update": "k_update"}
+                "ql": "k_lmin", "apply": "k_vec", "update": "k_update"}
 
 
 def kernel_work(name, stats, cfg, n_an, mixed):
@@ -53,13 +53,14 @@ def kernel_work(name, stats, cfg, n_an, mixed):
               mode (the three-term split's extra products are not counted),
               FP64 otherwise;
     apply:    T = V f V^T (2 k^3) and overline_w = Pa b (4 k^2) per analysis,
-              FP64 MFMA; the eigendecomposition itself (tridiag, QL, the
-              eigenvector accumulation) is excluded from F and reported as a
-              time share;
+              FP64 MFMA; the reduction to tridiagonal form and the other work
+              of the inverse square root are excluded from F and reported as
+              a time share;
     update:   Xa = Xb trans, 2 k^2 m flops, HBM-bound: Xb read and Xa written
               (2 s_x k m bytes, s_x = 4 for the FP32 state of the mixed form,
               8 for FP64) plus the means (16 m bytes) per analysis;
-    select, tridiag, ql: no F (index work, eigendecomposition).
+    select, tridiag, ql: no F (index work, the tridiagonal form and its
+              smallest eigenvalue).
     The FP64 vector and FP64 matrix peaks of MI355X are equal (78.6 TFLOP/s)."""
     k, m = cfg.k, cfg.n
     if name == "products":
@@ -263,7 +264,7 @@ def make_line(args, cfg, n_a, n_obs_rows, res, acc, cpu):
         "kernel_ms": head["kernel_ms"],
         "kernel_ms_timed_steps": head.get("kernel_ms_overlapped"),
         "kernel_ms_note": ("HIP-event time of each kernel over the whole batch, from two extra "
-                           "steps with the eigensolver on one stream"
+                           "steps"
                            if "kernel_ms_overlapped" in head else
                            "HIP-event time of each kernel over the whole batch"),
         "roofline": roof,
@@ -316,8 +317,8 @@ def parse():
     ap.add_argument("--graph", action="store_true",
                     help="timed steps replay a captured hipGraph of the call")
     ap.add_argument("--eig-one-stream", action="store_true",
-                    help="time the steps with the eigensolver on one stream (transform_kernel "
-                         "2; the default overlaps two half-batches on two streams)")
+                    help="time the steps with transform_kernel 2 (the same kernels as the "
+                         "default, 0)")
     ap.add_argument("--copy-probe", action="store_true",
                     help="only copy 1 GiB device to device three times (the calibration "
                          "kernel of the HBM traffic counters) and exit")
@@ -439,9 +440,7 @@ def main():
                     kernel_ms=k_ms, stats=stats, flagged=flagged, xa=xa, axa=axa, nobsl=nob,
                     bucket_stats=bstats)
 
-    # timed steps: the eigensolver overlaps two half-batches on two streams
-    # (transform_kernel 0), so its kernels are timed one at a time in a short
-    # extra leg with the eigensolver on one stream (transform_kernel 2)
+    # per-kernel times and bucket statistics come from a short extra leg
     tk = 2 if args.eig_one_stream else 0
     res = {}
     modes = [args.mixed] + ([] if args.no_fp64 else [PREC_FP64])

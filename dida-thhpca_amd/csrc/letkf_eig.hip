@@ -1,59 +1,45 @@
-// letkf_eig.hip -- FP64 eigensolve + transform + update in three kernels.
+// letkf_eig.hip -- the transform of a batch of local analyses and the ensemble
+// update: tridiagonalisation, the QL list pass, the update, and the launches.
 //
-// The k x k matrices M = A + (k-1)/rho I of one batch of local analyses are
-// diagonalised by Householder tridiagonalisation and implicit QL with
-// Wilkinson shift (Golub & Van Loan Alg. 8.3.1, Sec. 8.3.5; Bowdler, Martin,
-// Reinsch & Wilkinson 1968), split so that every phase runs with the
-// parallelism it has:
+// The k x k matrices M = A + (k-1)/rho I of one batch are reduced to
+// tridiagonal form, and trans and overline_w follow from that form:
 //
 //   k_tridiag   one wavefront per matrix, lane r keeps row r of A in VGPRs;
 //               writes the reflectors, tau, and the tridiagonal (d, e)
-//   k_ql_log    one LANE per matrix (64 matrices per wavefront): the scalar
-//               QL recurrence, which is a serial chain per matrix; writes the
-//               eigenvalues and a log of the Givens rotations of every chase
-//   k_vec       one wavefront per matrix (k <= 64), lane r keeps row r of Z
-//               in VGPRs: Q = H_0 ... H_{k-3} by forward accumulation, the
-//               logged rotations applied in order (V = Q Z), then
-//               overline_w = V diag(1/lambda) V^T b and
-//               trans = V diag(sqrt((k-1)/lambda)) V^T + overline_w 1^T
-//               (letkf_core.F90:129-225) on f64 MFMA
+//   k_vec       trans and overline_w from the inverse square root of the
+//               tridiagonal form and its reflectors (letkf_sqrt.hip, with
+//               k_lmin before it for the reduced precisions' guard)
 //   k_update    the ensemble update xa = trans^T xb + axb, re-centred
 //               (xb_2_xa, letkf_compute.F90:259-329, or the per-level update
 //               of the vertical loop, letkf_compute.F90:501-552)
-// k = 65..128 runs k_tridiag128, k_ql_log<128>, k_vec128 and k_update128
-// with half rows per thread (256 threads per matrix).
+// k = 65..128 runs k_tridiag128 and k_update128 with half rows per thread
+// (256 threads per matrix).
 //
-// Matrices whose QL did not converge or whose rotation log overflowed are
-// flagged (status != 0) and appended to a device-side list; k_vec and
-// k_update skip them.  A second pass of k_ql_log, k_vec and k_update over
-// that list (list mode: a longer rotation log, more QL iterations) redoes
-// them from the stored tridiagonal form, with no host synchronisation.  An
-// analysis still flagged after it leaves xa = xb, axa = axb for its state and
-// NaN in trans/overline_w; the caller gets the count.
+// A matrix whose M is not positive definite, or not finite, is flagged
+// (status != 0) and appended to a device-side list; k_update skips it.  The
+// list pass then diagonalises it by implicit QL with Wilkinson shift (Golub &
+// Van Loan Alg. 8.3.1, Sec. 8.3.5; Bowdler, Martin, Reinsch & Wilkinson
+// 1968) from the stored tridiagonal form, with no host synchronisation:
+//
+//   k_ql_log    one LANE per matrix (64 matrices per wavefront): the scalar
+//               QL recurrence, which is a serial chain per matrix; writes the
+//               eigenvalues and a log of the Givens rotations of every chase
+//   k_rot       one wavefront per matrix (k <= 64; k_rot128 above), lane r
+//               keeps row r of Z in VGPRs: Q = H_0 ... H_{k-3} by forward
+//               accumulation, the logged rotations applied in order (V = Q Z),
+//               then overline_w = V diag(1/lambda) V^T b and
+//               trans = V diag(sqrt((k-1)/lambda)) V^T + overline_w 1^T
+//               (letkf_core.F90:129-225) on f64 MFMA
+// An analysis still flagged after it (QL not converged, or its rotation log
+// full) leaves xa = xb, axa = axb for its state and NaN in trans/overline_w;
+// the caller gets the count.  With the QL limits lowered from the environment
+// (EigParams::ql_first) the first pass is the QL recurrence for every matrix,
+// so that its flag paths can be tested.
 #include "letkf_device.h"
 #include "letkf_kernels.h"
+#include "letkf_eig.h"
 
 namespace dida {
-
-// The analysis of workgroup (or lane) `slot`: a = global index, ai = index of
-// the batch-local inputs (A, b, refl, tau, d, e), ar = index of the pass's own
-// scratch (rot, hdr, nchase, lam).  False when the slot holds no analysis.
-__device__ __forceinline__ bool eig_slot(const EigParams& p, long long slot, long long& a,
-                                         long long& ai, long long& ar) {
-  if (p.list) {
-    const int n = min(*p.list_n, p.list_cap);
-    if (slot >= n) return false;
-    a = p.list[slot];
-    ai = a - p.a0;
-    ar = slot;
-  } else {
-    if (slot >= p.n_an) return false;
-    a = p.a0 + slot;
-    ai = slot;
-    ar = slot;
-  }
-  return true;
-}
 
 __global__ void k_zero_ints(int* __restrict__ p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -80,16 +66,6 @@ __device__ __forceinline__ AnRows an_rows(const EigParams& p, long long a) {
     r.ek = min(r.sk + p.cube_nz - 1, p.nz);
   }
   return r;
-}
-
-// trans and overline_w of an analysis whose eigensolve failed on both passes
-__device__ void nan_transform(const EigParams& p, long long a) {
-  const int k = p.k;
-  const double nan = __longlong_as_double(0x7ff8000000000000LL);
-  if (p.trans_out)
-    for (int e = threadIdx.x; e < k * k; e += blockDim.x) p.trans_out[a * (long long)k * k + e] = nan;
-  if (p.w_out)
-    for (int e = threadIdx.x; e < k; e += blockDim.x) p.w_out[a * (long long)k + e] = nan;
 }
 
 // ---------------------------------------------------------------------------
@@ -408,12 +384,11 @@ __device__ __forceinline__ double block2_min(double v, double* red, int& slot) {
 }
 
 // ---------------------------------------------------------------------------
-// k_vec + k_update: the k_apply work in two kernels sized for two wavefronts
-// per SIMD.  k_vec forms V (Q accumulation, logged rotations), overline_w and
-// trans = T + overline_w 1^T with LDS staged in small chunks, and writes
-// trans in the register layout of the update's MFMA B operand over the
-// analysis' reflector block (consumed by then).  k_update streams the state
-// vectors of the analysis through that operand.
+// k_rot (list pass): V (Q accumulation, logged rotations), overline_w and
+// trans = T + overline_w 1^T with LDS staged in small chunks, trans written
+// in the register layout of the update's MFMA B operand over the analysis'
+// reflector block (consumed by then), as k_vec does.  k_update streams the
+// state vectors of the analysis through that operand.
 // ---------------------------------------------------------------------------
 // The rotations of positions 8B .. 8B+7 of a chase: the log holds whole
 // blocks of 8 positions (identity outside the chase), position i at ring
@@ -451,15 +426,9 @@ struct VecLds {
   static constexpr int N = (A > B ? (A > C ? A : C) : (B > C ? B : C));
 };
 
-// offset (in doubles) of tile (I, J) register r of lane l in a trans block
-template <int KMAX>
-__device__ __forceinline__ int tile_off(int I, int J, int r, int l) {
-  return ((I * (KMAX / 16) + J) * 4 + r) * 64 + l;
-}
-
 template <int KMAX>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
-void k_vec(EigParams p) {
+void k_rot(EigParams p) {
   constexpr int NB = KMAX / 8;
   constexpr int TT = KMAX / 16;
   constexpr int IPP = TT < 2 ? TT : 2;               // tile rows per pass
@@ -468,7 +437,7 @@ void k_vec(EigParams p) {
   static_assert(REFILL >= KMAX + 16 && REFILL % 64 == 0, "a refill covers any chase");
   __shared__ __align__(16) double sbuf[L::N];
   // stage C's vectors share one array with stage A's Gram matrices (16 x 16),
-  // which are dead by then: k_vec<64> then needs 11.4 KB of LDS, so eight of
+  // which are dead by then: k_rot<64> then needs 11.4 KB of LDS, so eight of
   // its workgroups and one of k_ql_log's (66.5 KB) fit a CU together
   constexpr int NSC = 5 * KMAX > 256 ? 5 * KMAX : 256;
   __shared__ double ssc[NSC], stau[KMAX];
@@ -1077,7 +1046,7 @@ void k_update(EigParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// k_vec128 + k_update128: k = 65..128 with the rows of Z in registers.
+// k_rot128 + k_update128: k = 65..128 with the rows of Z in registers.
 // 256 threads per matrix: thread t keeps half h = t / 128 (columns
 // 64h .. 64h+63) of row r = t % 128.  A chase that crosses the middle (lo < 64
 // <= hi) runs on the upper half first; its carry goes to the lower half
@@ -1270,7 +1239,7 @@ __device__ __forceinline__ double chase_half(double (&z)[64], double& ztop, int 
   return carry;
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_vec128(EigParams p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_rot128(EigParams p) {
   constexpr int KMAX = 128, LDV = KMAX + 1, NT = 256;
   constexpr int RING = 1024, REFILL = 512;
   __shared__ __align__(16) double sbuf[16 * LDV > 2 * (RING + 8) ? 16 * LDV : 2 * (RING + 8)];
@@ -1836,69 +1805,10 @@ static void launch_update(hipStream_t st, const EigParams& p, unsigned nb) {
   }
 }
 
-hipError_t launch_eig(hipStream_t st, const EigParams& p, hipEvent_t* ev) {
-  if (p.n_an <= 0) return hipSuccess;
-  const unsigned nb = (unsigned)p.n_an;
-  const unsigned nq = (unsigned)((p.n_an + 63) / 64);
-  auto mark = [&](int i) -> hipError_t { return ev ? hipEventRecord(ev[i], st) : hipSuccess; };
-  hipError_t e = mark(0);
-  if (e != hipSuccess) return e;
-  if (p.k <= 32) {
-    if (p.tridiag_lds) hipLaunchKernelGGL(k_tridiag_lds<32>, dim3(nb), dim3(64), 0, st, p);
-    else hipLaunchKernelGGL(k_tridiag<32>, dim3(nb), dim3(64), 0, st, p);
-    if ((e = mark(1)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_ql_log<32>, dim3(nq), dim3(64), 0, st, p);
-    if ((e = mark(2)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_vec<32>, dim3(nb), dim3(64), 0, st, p);
-    if ((e = mark(3)) != hipSuccess) return e;
-    if (has_state(p)) launch_update<32>(st, p, nb);
-  } else if (p.k <= 64) {
-    if (p.tridiag_lds) hipLaunchKernelGGL(k_tridiag_lds<64>, dim3(nb), dim3(64), 0, st, p);
-    else hipLaunchKernelGGL(k_tridiag<64>, dim3(nb), dim3(64), 0, st, p);
-    if ((e = mark(1)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_ql_log<64>, dim3(nq), dim3(64), 0, st, p);
-    if ((e = mark(2)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_vec<64>, dim3(nb), dim3(64), 0, st, p);
-    if ((e = mark(3)) != hipSuccess) return e;
-    if (has_state(p)) launch_update<64>(st, p, nb);
-  } else if (p.k <= 128) {
-    if (p.tridiag_lds) hipLaunchKernelGGL(k_tridiag_lds<128>, dim3(nb), dim3(128), 0, st, p);
-    else hipLaunchKernelGGL(k_tridiag128, dim3(nb), dim3(256), 0, st, p);
-    if ((e = mark(1)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_ql_log<128>, dim3(nq), dim3(64), 0, st, p);
-    if ((e = mark(2)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_vec128, dim3(nb), dim3(256), 0, st, p);
-    if ((e = mark(3)) != hipSuccess) return e;
-    if (has_state(p)) launch_update<128>(st, p, nb);
-  } else {
-    return hipErrorInvalidValue;
-  }
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  return mark(4);
-}
-
-// analyses [off, off + n) of the batch p: batch-local arrays offset, global
-// ones (status, states, trans_out, w_out) unchanged
-static EigParams eig_slice(const EigParams& p, long long off, long long n) {
-  EigParams q = p;
-  const long long kp = p.kp;
-  q.a0 = p.a0 + off;
-  q.n_an = n;
-  q.A = p.A + off * kp * kp;
-  q.b = p.b + off * kp;
-  q.refl = p.refl + off * kp * kp;
-  q.tau = p.tau + off * kp;
-  q.d = p.d + off * kp;
-  q.e = p.e + off * kp;
-  q.lam = p.lam + off * kp;
-  q.rot = p.rot + off * (long long)p.rot_cap;
-  q.hdr = p.hdr + off * (long long)p.hdr_cap;
-  q.nchase = p.nchase + off;
-  return q;
-}
-
-// one of the four split-eigensolver kernels (tridiagonalisation, QL,
-// eigenvectors + trans, update) over the batch p
+// one of the four stages over the batch p: tridiagonalisation; the guard's
+// smallest eigenvalue (reduced precision); trans and overline_w; update.  With
+// ql_first stages 1 and 2 are the list pass's kernels, the QL recurrence and
+// its rotations.
 template <int KMAX>
 static void launch_eig_stage_k(hipStream_t st, const EigParams& p, int stage) {
   const unsigned nb = (unsigned)p.n_an;
@@ -1907,13 +1817,15 @@ static void launch_eig_stage_k(hipStream_t st, const EigParams& p, int stage) {
     if (p.tridiag_lds) hipLaunchKernelGGL(k_tridiag_lds<KMAX>, dim3(nb), dim3(KMAX < 64 ? 64 : KMAX), 0, st, p);
     else if constexpr (KMAX == 128) hipLaunchKernelGGL(k_tridiag128, dim3(nb), dim3(256), 0, st, p);
     else hipLaunchKernelGGL(k_tridiag<KMAX>, dim3(nb), dim3(64), 0, st, p);
+  } else if (stage == 3) {
+    if (has_state(p)) launch_update<KMAX>(st, p, nb);
+  } else if (!p.ql_first) {
+    (void)launch_sqrt(st, p, stage == 1);
   } else if (stage == 1) {
     hipLaunchKernelGGL(k_ql_log<KMAX>, dim3(nq), dim3(64), 0, st, p);
-  } else if (stage == 2) {
-    if constexpr (KMAX == 128) hipLaunchKernelGGL(k_vec128, dim3(nb), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(k_vec<KMAX>, dim3(nb), dim3(64), 0, st, p);
-  } else if (has_state(p)) {
-    launch_update<KMAX>(st, p, nb);
+  } else {
+    if constexpr (KMAX == 128) hipLaunchKernelGGL(k_rot128, dim3(nb), dim3(256), 0, st, p);
+    else hipLaunchKernelGGL(k_rot<KMAX>, dim3(nb), dim3(64), 0, st, p);
   }
 }
 
@@ -1921,6 +1833,21 @@ static void launch_eig_stage(hipStream_t st, const EigParams& p, int stage) {
   if (p.k <= 32) launch_eig_stage_k<32>(st, p, stage);
   else if (p.k <= 64) launch_eig_stage_k<64>(st, p, stage);
   else launch_eig_stage_k<128>(st, p, stage);
+}
+
+hipError_t launch_eig(hipStream_t st, const EigParams& p, hipEvent_t* ev) {
+  if (p.n_an <= 0) return hipSuccess;
+  if (p.k > 128) return hipErrorInvalidValue;
+  for (int stage = 0; stage < 4; ++stage) {
+    if (ev) {
+      const hipError_t e = hipEventRecord(ev[stage], st);
+      if (e != hipSuccess) return e;
+    }
+    launch_eig_stage(st, p, stage);
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return ev ? hipEventRecord(ev[4], st) : hipSuccess;
 }
 
 hipError_t launch_zero_ints(hipStream_t st, int* p, int n) {
@@ -1940,47 +1867,19 @@ hipError_t launch_eig_rerun(hipStream_t st, const EigParams& p) {
   for (int stage = 1; stage < 4; ++stage) {
     if (p.k <= 32) {
       if (stage == 1) hipLaunchKernelGGL(k_ql_log<32>, dim3(nq), dim3(64), 0, st, p);
-      else if (stage == 2) hipLaunchKernelGGL(k_vec<32>, dim3(nb), dim3(64), 0, st, p);
+      else if (stage == 2) hipLaunchKernelGGL(k_rot<32>, dim3(nb), dim3(64), 0, st, p);
       else if (has_state(p)) launch_update<32>(st, p, nb);
     } else if (p.k <= 64) {
       if (stage == 1) hipLaunchKernelGGL(k_ql_log<64>, dim3(nq), dim3(64), 0, st, p);
-      else if (stage == 2) hipLaunchKernelGGL(k_vec<64>, dim3(nb), dim3(64), 0, st, p);
+      else if (stage == 2) hipLaunchKernelGGL(k_rot<64>, dim3(nb), dim3(64), 0, st, p);
       else if (has_state(p)) launch_update<64>(st, p, nb);
     } else {
       if (stage == 1) hipLaunchKernelGGL(k_ql_log<128>, dim3(nq), dim3(64), 0, st, p);
-      else if (stage == 2) hipLaunchKernelGGL(k_vec128, dim3(nb), dim3(256), 0, st, p);
+      else if (stage == 2) hipLaunchKernelGGL(k_rot128, dim3(nb), dim3(256), 0, st, p);
       else if (has_state(p)) launch_update<128>(st, p, nb);
     }
   }
   return hipGetLastError();
-}
-
-hipError_t launch_eig_pipelined(hipStream_t st, hipStream_t st2, hipEvent_t e_first,
-                                hipEvent_t e_join, const EigParams& p, hipEvent_t* ev) {
-  if (p.k > 128 || p.n_an < 2 * kEigPipeMinHalf) return launch_eig(st, p, ev);
-  // the QL recurrence holds a CU's LDS with one wavefront and leaves its other
-  // SIMDs idle; the second half of the batch starts on st2 once the first
-  // half's tridiagonalisation is done, so its kernels run beside the first
-  // half's (tridiagonalisation beside QL, QL beside the eigenvectors)
-  const long long n1 = (p.n_an + 1) / 2;
-  const EigParams pa = eig_slice(p, 0, n1), pb = eig_slice(p, n1, p.n_an - n1);
-  auto mark = [&](int i) -> hipError_t { return ev ? hipEventRecord(ev[i], st) : hipSuccess; };
-  hipError_t e = mark(0);
-  if (e != hipSuccess) return e;
-  launch_eig_stage(st, pa, 0);
-  if ((e = hipEventRecord(e_first, st)) != hipSuccess) return e;
-  if ((e = hipStreamWaitEvent(st2, e_first, 0)) != hipSuccess) return e;
-  for (int stage = 0; stage < 4; ++stage) launch_eig_stage(st2, pb, stage);
-  if ((e = hipEventRecord(e_join, st2)) != hipSuccess) return e;
-  if ((e = mark(1)) != hipSuccess) return e;
-  launch_eig_stage(st, pa, 1);
-  if ((e = mark(2)) != hipSuccess) return e;
-  launch_eig_stage(st, pa, 2);
-  if ((e = mark(3)) != hipSuccess) return e;
-  launch_eig_stage(st, pa, 3);
-  if ((e = hipStreamWaitEvent(st, e_join, 0)) != hipSuccess) return e;
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  return mark(4);
 }
 
 }  // namespace dida

@@ -252,20 +252,6 @@ struct EigScratch {
   // scratch (its longer rotation log, chase headers, eigenvalues)
   DevBuf flags, rr_rot, rr_hdr, rr_nchase, rr_lam;
   std::vector<int> st_host;
-  // second stream and events of the k = 65..128 half-batch pipeline, created
-  // on first use (default priority)
-  hipStream_t st2 = nullptr;
-  hipEvent_t e_first = nullptr, e_join = nullptr;
-  void release_streams() {
-    if (st2) {
-      (void)hipStreamSynchronize(st2);
-      (void)hipStreamDestroy(st2);
-      st2 = nullptr;
-    }
-    if (e_first) (void)hipEventDestroy(e_first);
-    if (e_join) (void)hipEventDestroy(e_join);
-    e_first = e_join = nullptr;
-  }
 };
 
 
@@ -297,8 +283,7 @@ int products_band() {
 // bytes of split-eigensolver scratch per analysis
 size_t eig_bytes_per_analysis(int k) {
   const int kp = kp_of(k);
-  return sizeof(double) * ((size_t)kp * kp + 4 * kp) + 16 * (size_t)rot_cap_of(k) +
-         16 * (size_t)kHdrCapPerK * k + sizeof(int);
+  return sizeof(double) * ((size_t)kp * kp + 4 * kp);
 }
 
 // QL iterations per eigenvalue before a matrix is flagged (first pass; the
@@ -316,15 +301,18 @@ size_t rerun_bytes_per_slot(int k) {
          sizeof(double) * kp + sizeof(int);
 }
 
-// Optional positive integer from the environment (0 when unset).  The
-// eigensolver's limits can be lowered this way to make the flag paths run:
-// DIDA_ROT_CAP / DIDA_QL_MAXITER (first pass), DIDA_RERUN_ROT_CAP /
-// DIDA_RERUN_MAXITER (list pass).
+// Optional positive integer from the environment (0 when unset).  The QL
+// recurrence's limits can be lowered this way to make the flag paths run:
+// DIDA_ROT_CAP / DIDA_QL_MAXITER (first pass, which is then the QL recurrence
+// for every analysis), DIDA_RERUN_ROT_CAP / DIDA_RERUN_MAXITER (list pass).
 int env_int(const char* name) {
   const char* e = std::getenv(name);
   if (!e || !*e) return 0;
   return std::max(0, std::atoi(e));
 }
+
+// The first pass takes the QL recurrence only where its limits are set.
+bool ql_first() { return env_int("DIDA_ROT_CAP") || env_int("DIDA_QL_MAXITER"); }
 
 // Sizes every eigensolver buffer for batches of up to n analyses (the list
 // pass's too), so that the launches of a call allocate nothing.
@@ -336,9 +324,11 @@ int eig_prepare(EigScratch& s, int k, long long n) {
   RC_TRY(s.d.ensure(sizeof(double) * n * kp));
   RC_TRY(s.e.ensure(sizeof(double) * n * kp));
   RC_TRY(s.lam.ensure(sizeof(double) * n * kp));
-  RC_TRY(s.rot.ensure((size_t)16 * n * rot_cap_of(k)));
-  RC_TRY(s.hdr.ensure((size_t)16 * n * kHdrCapPerK * k));
-  RC_TRY(s.nchase.ensure(sizeof(int) * n));
+  if (ql_first()) {
+    RC_TRY(s.rot.ensure((size_t)16 * n * rot_cap_of(k)));
+    RC_TRY(s.hdr.ensure((size_t)16 * n * kHdrCapPerK * k));
+    RC_TRY(s.nchase.ensure(sizeof(int) * n));
+  }
   RC_TRY(s.flags.ensure(sizeof(int) * (2 + cap)));
   RC_TRY(s.rr_rot.ensure((size_t)16 * cap * 2 * rot_cap_of(k)));
   RC_TRY(s.rr_hdr.ensure((size_t)16 * cap * 2 * kHdrCapPerK * k));
@@ -368,9 +358,12 @@ int prepare_eig(EigScratch& s, const XformParams& xp, EigParams& ep) {
   RC_TRY(s.d.ensure(sizeof(double) * n * kp));
   RC_TRY(s.e.ensure(sizeof(double) * n * kp));
   RC_TRY(s.lam.ensure(sizeof(double) * n * kp));
-  RC_TRY(s.rot.ensure((size_t)16 * n * rot_cap));
-  RC_TRY(s.hdr.ensure((size_t)16 * n * hdr_cap));
-  RC_TRY(s.nchase.ensure(sizeof(int) * n));
+  const bool ql = ql_first();
+  if (ql) {
+    RC_TRY(s.rot.ensure((size_t)16 * n * rot_cap));
+    RC_TRY(s.hdr.ensure((size_t)16 * n * hdr_cap));
+    RC_TRY(s.nchase.ensure(sizeof(int) * n));
+  }
   const long long rcap = rerun_cap_of(k, n);
   if (s.flags.bytes < sizeof(int) * (2 + rcap))
     return set_error(DIDA_ERR_STATE, "eigensolver flags not set up for this batch");
@@ -380,6 +373,7 @@ int prepare_eig(EigScratch& s, const XformParams& xp, EigParams& ep) {
   ep.kp = kp;
   ep.inflation = xp.inflation;
   ep.guard = xp.guard;
+  ep.ql_first = ql;
   ep.max_iter = env_int("DIDA_QL_MAXITER") ? env_int("DIDA_QL_MAXITER") : kQlMaxIter;
   ep.flag_n = s.flags.as<int>();
   ep.flag_total = s.flags.as<int>() + 1;
@@ -466,21 +460,9 @@ int rerun_flagged(hipStream_t st, EigScratch& s, const EigParams& ep) {
   return DIDA_OK;
 }
 
-// The half-batch pipeline's second stream and its fork / join events (a
-// captured call records them as graph dependencies).
-int eig_second_stream(EigScratch& s) {
-  if (s.st2) return DIDA_OK;
-  HIP_TRY(hipStreamCreateWithFlags(&s.st2, hipStreamNonBlocking));
-  HIP_TRY(hipEventCreateWithFlags(&s.e_first, hipEventDisableTiming));
-  HIP_TRY(hipEventCreateWithFlags(&s.e_join, hipEventDisableTiming));
-  return DIDA_OK;
-}
-
 // Transform + update of analyses [xp.a0, xp.a0 + xp.n_an): the split
 // eigensolver, then its list pass over the analyses it flagged; mode 1 runs
-// only the single kernel (k <= 64).  Mode 0 runs batches of 2 kEigPipeMinHalf
-// analyses or more as two half-batches on two streams; mode 2 keeps the split
-// eigensolver on st (each kernel timed by itself).
+// only the single kernel (k <= 64).
 // kev: null, or 5 events for the split kernels (recorded only if *split is set)
 int run_transform(hipStream_t st, EigScratch& s, const XformParams& xp, int mode,
                   hipEvent_t* kev = nullptr, bool* split = nullptr) {
@@ -493,12 +475,7 @@ int run_transform(hipStream_t st, EigScratch& s, const XformParams& xp, int mode
   EigParams ep;
   RC_TRY(prepare_eig(s, xp, ep));
   HIP_TRY(launch_zero_ints(st, ep.flag_n, 1));
-  if (mode == 0 && xp.n_an >= 2 * kEigPipeMinHalf) {
-    RC_TRY(eig_second_stream(s));
-    HIP_TRY(launch_eig_pipelined(st, s.st2, s.e_first, s.e_join, ep, kev));
-  } else {
-    HIP_TRY(launch_eig(st, ep, kev));
-  }
+  HIP_TRY(launch_eig(st, ep, kev));
   if (split) *split = true;
   return rerun_flagged(st, s, ep);
 }
@@ -733,7 +710,6 @@ int dida_letkf_create(const dida_letkf_config* cfg, dida_letkf_handle** out) {
 int dida_letkf_destroy(dida_letkf_handle* h) {
   if (!h) return DIDA_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  h->eig.release_streams();
   DevBuf* bufs[] = {&h->glat, &h->glon, &h->o_lat, &h->o_lon, &h->o_rowptr, &h->o_yb64,
                     &h->o_dep, &h->o_rinv64, &h->o_vco, &h->key_in, &h->key_out, &h->val_in,
                     &h->val_out, &h->hist, &h->bin_start, &h->sort_tmp, &h->s_cos, &h->s_sin,
@@ -1110,8 +1086,6 @@ static int prepare_call(dida_letkf_handle* h) {
     h->nobsl_host.assign(h->n_an, 0);
   }
   RC_TRY(eig_prepare(h->eig, c.k, mb * h->nzc));
-  if (c.transform_kernel == 0 && mb * h->nzc >= 2 * kEigPipeMinHalf)
-    RC_TRY(eig_second_stream(h->eig));
   if (h->opt_schedule == 1 && !h->tiled) {
     RC_TRY(h->b_order.ensure(sizeof(int) * mb * h->nzc));
     RC_TRY(h->b_blk.ensure(sizeof(long long) * std::max(bucket_blk_elems((int)mb), 1LL)));
@@ -1626,9 +1600,8 @@ static void drop_graph(dida_letkf_handle* h) {
   h->gkey.clear();
 }
 
-// Captures the call's launches (no timing events; the half-batch pipeline's
-// second stream joins the capture through its fork / join events) unless
-// the graph of an identical earlier call exists, and launches the graph.
+// Captures the call's launches (no timing events) unless the graph of an
+// identical earlier call exists, and launches the graph.
 static int graph_call(dida_letkf_handle* h, const StateArgs& sa, float& ms) {
   hipStream_t st = h->stream;
   if (!st) return set_error(DIDA_ERR_STATE, "graph mode needs a non-null stream");
@@ -1903,9 +1876,11 @@ int core_layout(CoreBufs& cb, EigScratch& es, int k, long long n_an, long long n
   add(es.d, 8 * n * kp);
   add(es.e, 8 * n * kp);
   add(es.lam, 8 * n * kp);
-  add(es.rot, 16 * n * (size_t)rot_cap_of(k));
-  add(es.hdr, 16 * n * (size_t)(kHdrCapPerK * k));
-  add(es.nchase, 4 * n);
+  if (ql_first()) {
+    add(es.rot, 16 * n * (size_t)rot_cap_of(k));
+    add(es.hdr, 16 * n * (size_t)(kHdrCapPerK * k));
+    add(es.nchase, 4 * n);
+  }
   add(es.flags, 4 * (2 + cap));
   add(es.rr_rot, 16 * cap * (size_t)(2 * rot_cap_of(k)));
   add(es.rr_hdr, 16 * cap * (size_t)(2 * kHdrCapPerK * k));
@@ -2030,6 +2005,7 @@ void release_core(CoreBufs& cb, EigScratch& es) {
   size_t sizes[kCoreMaxBufs];
   const int nb = core_layout(cb, es, 2, 1, 1, DIDA_PREC_BF16X3, bufs, sizes);
   for (int i = 0; i < nb; ++i) bufs[i]->release();
+  for (DevBuf* b : {&es.rot, &es.hdr, &es.nchase}) b->release();
 }
 
 // The drop-in letkf_core_ is called once per local analysis (64,800 times a
@@ -2083,7 +2059,6 @@ int dida_letkf_core_batched(int k, long long n_an, const long long* row_ptr, con
   const int rc = core_run(st, cb, es, 0, k, n_an, row_ptr, hxens, rdiaginv, dep, rloc, trans,
                           overline_w, inflation, precision, status);
   (void)hipStreamSynchronize(st);
-  es.release_streams();
   release_core(cb, es);
   (void)hipStreamDestroy(st);
   return rc;

@@ -228,8 +228,8 @@ struct EigParams {
   int guard;
   int max_iter;             // QL iterations per eigenvalue before the matrix is flagged
   long long a0, n_an;
-  // Flag list.  First pass (list == NULL): k_ql_log appends every analysis it
-  // flags to flag_list (global index, at most flag_cap entries; *flag_n
+  // Flag list.  First pass (list == NULL): k_vec (or k_ql_log, ql_first)
+  // appends every analysis it flags to flag_list (global index, at most flag_cap entries; *flag_n
   // counts all of them, *flag_total accumulates over the batches of a call).
   // Rerun pass (list != NULL): the kernels take analysis list[slot] for
   // slot < min(*list_n, list_cap); batch-local inputs (d, e, refl, tau, b) are
@@ -249,10 +249,13 @@ struct EigParams {
   double* tau;              // batch-local, kp
   double* d;                // batch-local, kp (tridiagonal diagonal)
   double* e;                // batch-local, kp (subdiagonal)
-  double* lam;              // batch-local, kp (eigenvalues of A)
+  double* lam;              // batch-local, kp: the smallest eigenvalue of A or 0 (k_lmin);
+                            // k_ql_log: all eigenvalues
   double2* rot;             // batch-local, rot_cap Givens (c, s) per analysis
   int4* hdr;                // batch-local, hdr_cap chases (lo, hi, off) per analysis
   int rot_cap, hdr_cap;
+  int ql_first;             // the first pass is the QL recurrence (rot, hdr, nchase sized for
+                            // the batch) instead of k_vec
   int tridiag_lds;          // k <= 64: tridiagonalise in LDS (1) or in VGPRs (0)
   int* nchase;              // batch-local
   int* status;              // global index
@@ -387,16 +390,10 @@ hipError_t launch_zero_halo(hipStream_t st, double* x, int nlat, int nlon, int h
 hipError_t launch_eig(hipStream_t st, const EigParams& p, hipEvent_t* ev = nullptr);
 // second pass over the analyses the first flagged (p.list / p.list_n / p.list_cap)
 hipError_t launch_eig_rerun(hipStream_t st, const EigParams& p);
+// the guard's smallest eigenvalue (guard_pass; nothing without p.guard), or
+// trans and overline_w, of the batch p from its tridiagonal form
+hipError_t launch_sqrt(hipStream_t st, const EigParams& p, bool guard_pass);
 hipError_t launch_zero_ints(hipStream_t st, int* p, int n);
-// k = 65..128 batches of at least 2 kEigPipeMinHalf analyses: the batch in two
-// halves, the second on st2 (ordered after the first half's
-// tridiagonalisation, joined back into st through e_join); ev as above, with
-// the first half's kernel boundaries (the second half's kernels run beside
-// them).  Smaller batches and k <= 64 take launch_eig on st.
-constexpr long long kEigPipeMinHalf = 1024;
-hipError_t launch_eig_pipelined(hipStream_t st, hipStream_t st2, hipEvent_t e_first,
-                                hipEvent_t e_join, const EigParams& p, hipEvent_t* ev = nullptr);
-
 // Entry (r, c) of one analysis' A, whose slot holds kp * kp doubles.  FP64:
 // column-major.  a_f32 (the BF16 products, kp = 32 or 64): the FP32 sums in
 // the products' tile order, column-major in the first half of the slot,

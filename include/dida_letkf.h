@@ -91,13 +91,10 @@ typedef struct dida_letkf_config {
     double p0, ptop;
     int keep_transforms;    /* keep trans/overline_w of every analysis */
     int max_batch_columns;  /* 0 = automatic */
-    int transform_kernel;   /* 0: split eigensolver (tridiagonalisation,
-                               lane-per-matrix QL, rotation apply), a batch
-                               of 2048 analyses or more as two half-batches
-                               on two streams; 1: the single-kernel
-                               transform (k <= 64); 2: the split eigensolver
-                               on the caller's stream only (its kernels
-                               timed one at a time) */
+    int transform_kernel;   /* 0, 2: split transform (tridiagonalisation, then
+                               the inverse square root of the tridiagonal
+                               form); 1: the single-kernel transform
+                               (k <= 64) */
     int products_kernel;    /* 0: automatic (= 1); 1: one selection list per
                                analysis; 2: tiles of 8 analyses sharing their
                                LDS-staged union of obs rows (horizontal loop,
@@ -122,13 +119,12 @@ typedef struct dida_letkf_stats {
     double ms_transform;    /* device time, eigensolve + transform + update */
     double ms_total;        /* device time of the whole call */
     double ms_tridiag;      /* of ms_transform: Householder tridiagonalisation kernel */
-    double ms_ql;           /* of ms_transform: QL recurrence kernel */
-    double ms_apply;        /* of ms_transform: eigenvector and transform kernel (k <= 64
-                               with the fused kernel: also the update) */
+    double ms_ql;           /* of ms_transform: smallest eigenvalue for the guard of the
+                               reduced precisions */
+    double ms_apply;        /* of ms_transform: inverse square root and transform kernel */
     double ms_update;       /* of ms_transform: ensemble update kernel (0 when fused) */
-    int n_rerun;            /* analyses the eigensolver's first pass flagged (QL not
-                               converged in 30 iterations, or its rotation log full)
-                               and its list pass redid */
+    int n_rerun;            /* analyses the transform's first pass flagged (M not positive
+                               definite or not finite) and its list pass redid by QL */
     /* Products schedule.  Length buckets over the local obs count p of a
      * column: [0] p = 0, [1] 1..256, [2] 257..512, ... [6] 4097..8192, [7] more. */
     int schedule;                    /* 1: buckets + persistent work queue; 0: column order */

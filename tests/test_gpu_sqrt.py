@@ -1,0 +1,105 @@
+"""GPU tests of the transform from the tridiagonal form (k_vec): the inverse
+square root by poles, the tiled resolvent sums and the blocked two-sided
+product, at the edges of its 16-wide tiles and pole groups.
+
+Tolerance: the reduction to tridiagonal form and the reference's
+eigendecomposition are each backward stable, an error of up to k eps |A| in A,
+hence up to k eps kappa / 2 relative to the largest entry of T (kappa the ratio
+of the largest eigenvalue of M to (k-1)/rho): max(1e-10, k eps kappa) for the
+two together, and twice that for overline_w = T T b / (k-1).
+"""
+import os
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    torch.cuda.set_device(0)
+
+
+def _case(k, p, scale, seed):
+    rng = np.random.default_rng(seed)
+    y = scale * rng.standard_normal((k, p)) * np.exp(-0.1 * np.arange(p))[None, :]
+    y -= y.mean(axis=0, keepdims=True)
+    return (y, (1.0 / rng.uniform(0.5, 2.0, p) ** 2).astype(np.float32), rng.standard_normal(p),
+            rng.uniform(0.1, 1.0, p))
+
+
+def _kappa(c, rho):
+    y, rinv, _, rloc = c
+    k = y.shape[0]
+    return 1.0 + np.linalg.eigvalsh((y * (rinv * rloc)) @ y.T).max() * rho / (k - 1)
+
+
+# k: 1 and 2 reflectors, the tile edges (one tile, a tile and one row, whole
+# tiles), the three kernel widths; scales give kappa from 1 to ~1e9, 8 to ~45
+# poles (one to three groups of 16)
+@pytest.mark.parametrize("k", [2, 3, 4, 15, 16, 17, 18, 19, 31, 32, 33, 34, 35, 48, 49, 63, 64,
+                               65, 66, 80, 81, 96, 113, 127, 128])
+def test_transform_edges(k):
+    import orc
+    from dida_letkf import engine
+    rho = 1.13
+    cases = [_case(k, p, s, 1000 * k + i) for i, (p, s) in enumerate(
+        [(0, 1.0), (1, 1.0), (40, 0.05), (60, 1.0), (60, 30.0), (60, 1e3), (60, 2e4)])]
+    args = [[c[i] for c in cases] for i in range(4)]
+    t, w, st = engine.letkf_core_batched(*args, inflation_factor=rho)
+    assert (st == 0).all()
+    old = os.environ.get("DIDA_QL_MAXITER")
+    os.environ["DIDA_QL_MAXITER"] = "30"              # the QL recurrence for every analysis
+    try:
+        tq, wq, sq = engine.letkf_core_batched(*args, inflation_factor=rho)
+    finally:
+        os.environ.pop("DIDA_QL_MAXITER")
+        if old is not None:
+            os.environ["DIDA_QL_MAXITER"] = old
+    assert (sq == 0).all()
+    for i, c in enumerate(cases):
+        kap = _kappa(c, rho) if c[0].shape[1] else 1.0
+        tol = max(1e-10, k * np.finfo(float).eps * kap)
+        t_o, w_o, _ = orc.letkf_core(*c, inflation_factor=rho)
+        for tt, ww in ((t[i], w[i]), (tq[i], wq[i])):
+            e_t = np.abs(tt - t_o).max() / np.abs(t_o).max()
+            e_w = np.abs(ww - w_o).max() / max(1.0, np.abs(w_o).max())
+            print(k, i, "kappa %.2g" % kap, e_t, e_w, flush=True)
+            assert e_t < tol and e_w < 2 * tol
+
+
+@pytest.mark.parametrize("k", [20, 40, 100])
+def test_weak_and_indefinite(k):
+    """Negative R^-1 makes A indefinite.  Where M stays positive definite (its
+    smallest eigenvalue far below (k-1)/rho) the first pass still gives the
+    transform; where it does not, the list pass's QL takes the matrix, with the
+    NaN of the square root of a negative eigenvalue.  (Against numpy's eigh: the
+    oracle forms sqrt(R^-1), which is NaN here.)"""
+    from dida_letkf import engine
+    rng = np.random.default_rng(k)
+    y = rng.standard_normal((k, 5))
+    y -= y.mean(axis=0, keepdims=True)
+    dep, rloc = rng.standard_normal(5), np.ones(5)
+    top = np.linalg.eigvalsh(y @ y.T).max()
+    cases, want = [], []
+    for f in (0.05, 0.2, 0.7, 0.97, 1.5):             # smallest eigenvalue (1 - f) (k-1)
+        cases.append((y, np.full(5, -f * (k - 1) / top, np.float32), dep, rloc))
+        want.append(f < 1.0)
+    t, w, st = engine.letkf_core_batched(*[[c[i] for c in cases] for i in range(4)])
+    for i, (yy, rinv, d, _) in enumerate(cases):
+        wy = yy * rinv.astype(np.float64)
+        lam, v = np.linalg.eigh(wy @ yy.T)
+        lam = lam + (k - 1)
+        if want[i]:
+            w_o = v @ ((v.T @ (wy @ d)) / lam)
+            t_o = (v * np.sqrt((k - 1) / lam)) @ v.T + w_o[:, None]
+            # kappa / (1 - f) <= 40 here: rounding, amplified 40 times
+            assert st[i] == 0
+            assert np.abs(t[i] - t_o).max() < 1e-10 * np.abs(t_o).max()
+            assert np.abs(w[i] - w_o).max() < 1e-10 * max(1.0, np.abs(w_o).max())
+        else:
+            assert np.isnan(t[i]).all()
