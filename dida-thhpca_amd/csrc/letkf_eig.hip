@@ -94,129 +94,138 @@ __device__ __forceinline__ double pick_column(const double (&arow)[N], int c) {
   return x;
 }
 
-// k = 64 is capped at 168 registers (three wavefronts per SIMD: the kernel is
-// bound by the latency of its per-step reductions and LDS round trips, and a
-// few spilled scalars cost less than the third wavefront gains)
+// Sum over the KMAX lanes of a matrix (all lanes active): rows of 16 on DPP,
+// then the rows by shuffles.
 template <int KMAX>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KMAX == 64 ? 3 : 2)))
+__device__ __forceinline__ double matrix_sum(double v) {
+  v += dpp_d<0xB1>(v);     // quad_perm [1,0,3,2]
+  v += dpp_d<0x4E>(v);     // quad_perm [2,3,0,1]
+  v += dpp_d<0x141>(v);    // row_half_mirror
+  v += dpp_d<0x140>(v);    // row_mirror
+  v += __shfl_xor(v, 16, 64);
+  return KMAX == 64 ? v + __shfl_xor(v, 32, 64) : v;
+}
+
+// k = 64: one matrix per wavefront; k <= 32: two, one per half (with one, half
+// the lanes had no row).  Per step the products and the update take v and w
+// as row broadcasts of the FMA (bcast_dot8, bcast_axpy8): w and v go through
+// LDS once, and each lane reads the NT entries of them that its row of 16
+// broadcasts.  Read entry by entry from LDS, the four SIMDs' 48 broadcast
+// reads a step bound the kernel; now VALU issue does (14.8k instructions per
+// wavefront, 6.1k of them FMAs).  64,800 matrices of k = 64: 3.25 -> 2.25 ms,
+// the same bits; 2,073,600 of k = 32: 37.5 -> 11.9 ms.
+template <int KMAX>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KMAX == 64 ? 3 : 4)))
 void k_tridiag(EigParams p) {
-  constexpr int NB = KMAX / 8;
-  __shared__ __align__(16) double sv[KMAX];
-  __shared__ __align__(16) double sw[KMAX];
-  __shared__ double se_s[KMAX + 1], st_s[KMAX + 1];
+  constexpr int NT = KMAX / 16, MPW = 64 / KMAX;
+  __shared__ double sv[64], sw[64];
+  __shared__ double se_s[64], st_s[64];
   __shared__ double sxn[64];             // column j+1 after step j's update
-  const int lane = threadIdx.x;
-  const long long a = p.a0 + blockIdx.x;
-  if (a >= p.a0 + p.n_an) return;
-  const long long al = a - p.a0;
+  const int lane = threadIdx.x, r = lane & (KMAX - 1), m0 = lane - r;
+  const long long nal = (long long)blockIdx.x * MPW + (m0 ? 1 : 0);
+  // a wavefront's second matrix past the batch's end repeats the last one,
+  // storing nothing
+  const bool valid = MPW == 1 || nal < p.n_an;
+  const long long al = valid ? nal : p.n_an - 1;
   const int k = p.k, kp = p.kp;
   const double* __restrict__ Ag = p.A + al * (long long)kp * kp;
   double* __restrict__ refl = p.refl + al * (long long)kp * kp;
-  const bool in_r = lane < k;
+  const bool in_r = r < k;
+  const double* const svr = sv + m0 + (lane & 15);
+  const double* const swr = sw + m0 + (lane & 15);
 
   double arow[KMAX];
   if (p.a_f32) {
     // FP32 in tile order (a_entry; kp = KMAX): one base address per lane and
-    // a constant offset per column, every load unconditional and in bounds
-    // (lanes past kp read position 0), then a select
-    const float* __restrict__ Af =
-        reinterpret_cast<const float*>(Ag) + a_tile_pos(lane < KMAX ? lane : 0, KMAX);
+    // a constant offset per column, every load unconditional and in bounds,
+    // then a select
+    const float* __restrict__ Af = reinterpret_cast<const float*>(Ag) + a_tile_pos(r, KMAX);
     float av[KMAX];
 #pragma unroll
     for (int c = 0; c < KMAX; ++c) av[c] = Af[a_tile_pos(c, KMAX) * KMAX];
 #pragma unroll
     for (int c = 0; c < KMAX; ++c) arow[c] = (in_r && c < k) ? (double)av[c] : 0.0;
   } else {
+    // (kp = KMAX here too) the pins keep the loads out of the selects: a load
+    // under the select's test waits for the one before it
 #pragma unroll
-    for (int c = 0; c < KMAX; ++c)
-      arow[c] = (in_r && c < k) ? Ag[(long long)c * kp + lane] : 0.0;
+    for (int c = 0; c < KMAX; ++c) arow[c] = Ag[(long long)c * KMAX + r];
+#pragma unroll
+    for (int c = 0; c < KMAX; ++c) pin(arow[c]);
+#pragma unroll
+    for (int c = 0; c < KMAX; ++c) arow[c] = (in_r && c < k) ? arow[c] : 0.0;
   }
-  double xcol = arow[0];
+  sxn[lane] = arow[0];
+  se_s[lane] = st_s[lane] = 0.0;
+  __syncthreads();
 
   for (int j = 0; j + 2 < k; ++j) {
-    const bool act = in_r && lane > j;
+    const bool act = in_r && r > j;
+    const double xcol = sxn[lane], x0 = sxn[m0 + j + 1];
     const double x = act ? xcol : 0.0;
-    const double x0 = readlane_d(xcol, j + 1);
-    const double rest = wave_sum_full((act && lane > j + 1) ? x * x : 0.0);
+    const double rest = matrix_sum<KMAX>((act && r > j + 1) ? x * x : 0.0);
     __builtin_amdgcn_sched_barrier(0);
-    if (rest == 0.0) {
-      // column already in tridiagonal form; column j+1 goes through LDS
-      sxn[lane] = pick_column(arow, j + 1);
-      if (lane < KMAX) refl[(long long)j * kp + lane] = 0.0;
-      if (lane == 0) { se_s[j] = x0; st_s[j] = 0.0; }
-      __syncthreads();
-      xcol = sxn[lane];
-      continue;
-    }
+    // a column already in tridiagonal form (rest = 0) takes the same path with
+    // v = 0 and tau = 0: the update is then exactly the identity
+    const bool none = rest == 0.0;
     const double nrm = sqrt(rest + x0 * x0);
     const double alpha = (x0 >= 0.0) ? -nrm : nrm;
     const double v0 = x0 - alpha;
-    const double tau = 2.0 / (rest + v0 * v0);
-    const double v = act ? ((lane == j + 1) ? v0 : x) : 0.0;
-    if (lane < KMAX) sv[lane] = v;
+    const double tau = none ? 0.0 : 2.0 / (rest + v0 * v0);
+    const double v = (act && !none) ? ((r == j + 1) ? v0 : x) : 0.0;
+    sv[lane] = v;
     __syncthreads();
-    // p = tau A v over the trailing columns (sv is zero for c <= j); four
-    // partial sums, one block of 8 columns in flight at a time
-    double pr0 = 0.0, pr1 = 0.0, pr2 = 0.0, pr3 = 0.0;
+    double vt[NT];
 #pragma unroll
-    for (int B = 0; B < NB; ++B) {
-      if (8 * B + 7 <= j) continue;
-      pr0 = fma(arow[8 * B + 0], sv[8 * B + 0], pr0);
-      pr1 = fma(arow[8 * B + 1], sv[8 * B + 1], pr1);
-      pr2 = fma(arow[8 * B + 2], sv[8 * B + 2], pr2);
-      pr3 = fma(arow[8 * B + 3], sv[8 * B + 3], pr3);
-      pr0 = fma(arow[8 * B + 4], sv[8 * B + 4], pr0);
-      pr1 = fma(arow[8 * B + 5], sv[8 * B + 5], pr1);
-      pr2 = fma(arow[8 * B + 6], sv[8 * B + 6], pr2);
-      pr3 = fma(arow[8 * B + 7], sv[8 * B + 7], pr3);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int t = 0; t < NT; ++t) vt[t] = svr[16 * t];
+    // p = tau A v over the trailing columns (v is zero for c <= j); four
+    // partial sums
+    double pr4[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (16 * t + 7 > j) bcast_dot8<0>(pr4, vt[t], arow + 16 * t);
+      if (16 * t + 15 > j) bcast_dot8<1>(pr4, vt[t], arow + 16 * t + 8);
     }
-    double pr = (pr0 + pr1) + (pr2 + pr3);
+    double pr = (pr4[0] + pr4[1]) + (pr4[2] + pr4[3]);
     pr = act ? pr * tau : 0.0;
-    const double K = 0.5 * tau * wave_sum_full(v * pr);
+    const double K = 0.5 * tau * matrix_sum<KMAX>(v * pr);
     __builtin_amdgcn_sched_barrier(0);
     const double wr = act ? pr - K * v : 0.0;
-    if (lane < KMAX) sw[lane] = wr;
+    sw[lane] = wr;
+    if (valid) refl[(long long)j * kp + r] = v;
+    if (r == 0) { se_s[m0 + j] = none ? x0 : alpha; st_s[m0 + j] = tau; }
     __syncthreads();
-    // rank-2 update A -= v w^T + w v^T, a block of 8 columns per LDS round
-    // trip (sv and sw are zero for c <= j); column j+1 goes through LDS after
-    // the whole update
+    // rank-2 update A -= v w^T + w v^T (v and w are zero for c <= j); column
+    // j+1 goes through LDS after the whole update
 #pragma unroll
-    for (int B = 0; B < NB; ++B) {
-      if (8 * B + 7 <= j) continue;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int c = 8 * B + t;
-        arow[c] = fma(-wr, sv[c], fma(-v, sw[c], arow[c]));
+    for (int t = 0; t < NT; ++t) {
+      const double wt = swr[16 * t];
+      if (16 * t + 7 > j) {
+        bcast_axpy8<0>(arow + 16 * t, wt, -v);
+        bcast_axpy8<0>(arow + 16 * t, vt[t], -wr);
       }
-      __builtin_amdgcn_sched_barrier(0);
+      if (16 * t + 15 > j) {
+        bcast_axpy8<1>(arow + 16 * t + 8, wt, -v);
+        bcast_axpy8<1>(arow + 16 * t + 8, vt[t], -wr);
+      }
     }
     sxn[lane] = pick_column(arow, j + 1);
-    if (lane < KMAX) refl[(long long)j * kp + lane] = v;
-    if (lane == 0) { se_s[j] = alpha; st_s[j] = tau; }
     __syncthreads();
-    xcol = sxn[lane];
   }
   // diagonal and the last subdiagonal entry
   double dr = 0.0, ek2 = 0.0;
 #pragma unroll
   for (int c = 0; c < KMAX; ++c) {
-    dr = (c == lane) ? arow[c] : dr;
+    dr = (c == r) ? arow[c] : dr;
     ek2 = (c == k - 2) ? arow[c] : ek2;
   }
-  ek2 = readlane_d(ek2, k - 1);
+  sxn[lane] = ek2;
   __syncthreads();
-  double* __restrict__ dg = p.d + al * kp;
-  double* __restrict__ eg = p.e + al * kp;
-  double* __restrict__ tg = p.tau + al * kp;
-  if (lane < KMAX) {
-    dg[lane] = in_r ? dr : 0.0;
-    double ev = 0.0, tv = 0.0;
-    if (lane + 2 < k) { ev = se_s[lane]; tv = st_s[lane]; }
-    else if (lane == k - 2) ev = ek2;
-    eg[lane] = ev;
-    tg[lane] = tv;
-  }
+  ek2 = sxn[m0 + k - 1];
+  if (!valid) return;
+  p.d[al * kp + r] = in_r ? dr : 0.0;
+  p.e[al * kp + r] = r == k - 2 ? ek2 : se_s[lane];
+  p.tau[al * kp + r] = st_s[lane];
 }
 
 // ---------------------------------------------------------------------------
@@ -1060,7 +1069,9 @@ void k_update(EigParams p) {
 // registers (thread t: row t % 128, the columns of parity h = t / 128, one
 // half per wavefront): the halves interleave, so both keep the same share of
 // the shrinking trailing matrix, and blocks of columns <= j (where v and w
-// are zero) are skipped.  A column already in tridiagonal form runs the same
+// are zero) are skipped.  v and w enter the FMAs as row broadcasts, as in
+// k_tridiag (64,800 matrices of k = 128: 34.3 -> 23.9 ms).  A column already
+// in tridiagonal form runs the same
 // step with v = 0 and tau = 0 (an exact identity update), so the loop has one
 // path and A stays in the same registers.  Three wavefronts per SIMD.  Same
 // outputs as k_tridiag.  Three barriers per step:
@@ -1145,19 +1156,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     const double tau = none ? 0.0 : 2.0 / (rest + v0 * v0);
     if (lane == 0) col[j + 1] = v0;
     const double vr = act ? col[r] : 0.0;
-    // partial p over this half (v_c = 0 for c <= j)
-    double p0 = 0.0, p1 = 0.0;
+    // partial p over this half (v_c = 0 for c <= j; row broadcasts as in
+    // k_tridiag, lane i of a row holding entry 2 (16 t + i) + h)
+    double vt[4];
 #pragma unroll
-    for (int B = 0; B < 8; ++B) {
-      if (16 * B + 14 + h <= j) continue;      // v is zero over these columns
+    for (int t = 0; t < 4; ++t) vt[t] = col[2 * (16 * t + (lane & 15)) + h];
+    double p4[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int c = 8 * B; c < 8 * B + 8; c += 2) {
-        p0 = fma(arow[c], col[2 * c + h], p0);
-        p1 = fma(arow[c + 1], col[2 * c + 2 + h], p1);
-      }
-      __builtin_amdgcn_sched_barrier(0);
+    for (int t = 0; t < 4; ++t) {
+      if (32 * t + 14 + h > j) bcast_dot8<0>(p4, vt[t], arow + 16 * t);
+      if (32 * t + 30 + h > j) bcast_dot8<1>(p4, vt[t], arow + 16 * t + 8);
     }
-    const double ph = p0 + p1;
+    const double ph = (p4[0] + p4[1]) + (p4[2] + p4[3]);
     if (in_r) spr[h][r] = ph;
     {
       const double vp = wave_sum_full(vr * ph);
@@ -1171,14 +1181,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     __syncthreads();
     // A -= v w^T + w v^T over this half (vr = wr = 0 in rows <= j)
 #pragma unroll
-    for (int B = 0; B < 8; ++B) {
-      if (16 * B + 14 + h <= j) continue;      // v and w are zero over these columns
-#pragma unroll
-      for (int c = 8 * B; c < 8 * B + 8; ++c) {
-        const int cg = 2 * c + h;
-        arow[c] = fma(-wr, col[cg], fma(-vr, sw[cg], arow[c]));
+    for (int t = 0; t < 4; ++t) {
+      const double wt = sw[2 * (16 * t + (lane & 15)) + h];
+      if (32 * t + 14 + h > j) {
+        bcast_axpy8<0>(arow + 16 * t, wt, -vr);
+        bcast_axpy8<0>(arow + 16 * t, vt[t], -wr);
       }
-      __builtin_amdgcn_sched_barrier(0);
+      if (32 * t + 30 + h > j) {
+        bcast_axpy8<1>(arow + 16 * t + 8, wt, -vr);
+        bcast_axpy8<1>(arow + 16 * t + 8, vt[t], -wr);
+      }
     }
     pass_column(j, nxt);
     if (h == 0) refl[(long long)j * kp + r] = vr;
@@ -1816,7 +1828,7 @@ static void launch_eig_stage_k(hipStream_t st, const EigParams& p, int stage) {
   if (stage == 0) {
     if (p.tridiag_lds) hipLaunchKernelGGL(k_tridiag_lds<KMAX>, dim3(nb), dim3(KMAX < 64 ? 64 : KMAX), 0, st, p);
     else if constexpr (KMAX == 128) hipLaunchKernelGGL(k_tridiag128, dim3(nb), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(k_tridiag<KMAX>, dim3(nb), dim3(64), 0, st, p);
+    else hipLaunchKernelGGL(k_tridiag<KMAX>, dim3(KMAX == 32 ? (nb + 1) / 2 : nb), dim3(64), 0, st, p);
   } else if (stage == 3) {
     if (has_state(p)) launch_update<KMAX>(st, p, nb);
   } else if (!p.ql_first) {

@@ -120,12 +120,6 @@ __global__ __launch_bounds__(64) void k_lmin(EigParams p) {
   if (t == 0 && al0 + mt < p.n_an) p.lam[(al0 + mt) * kp] = 0.5 * (lo + hi);
 }
 
-// Keeps x in registers here, in program order: the unrolled blocks below are
-// long runs of pure arithmetic, which the compiler otherwise gathers far from
-// their loads, and spills.
-__device__ __forceinline__ void pin(double& x) { asm volatile("" : "+v"(x)); }
-__device__ __forceinline__ void pin(d4& x) { asm volatile("" : "+v"(x)); }
-
 // ---------------------------------------------------------------------------
 // k_vec
 // ---------------------------------------------------------------------------
