@@ -442,20 +442,27 @@ __device__ __forceinline__ long long analysis_at(const ProdParams& p, long long 
 //      workers (3, 4) that ran.
 // Within a bucket segment the analyses an XCD runs are neighbours in the
 // grid and share their obs rows in that XCD's L2.
-template <int WPA, int SCHED, class Body>
+// LV > 1 (level loop): a visit covers up to LV consecutive levels of a column
+// (the column's nzc analyses are consecutive in the order list too), body
+// getting the first; positions and queue counters then count such units.
+template <int WPA, int SCHED, int LV = 1, class Body>
 __device__ __forceinline__ void for_analyses(const ProdParams& p, int lane, Body body) {
   static_assert(WPA == 1 || WPA == 4, "a wavefront or a workgroup per analysis");
+  const int upc = LV > 1 ? (p.nzc + LV - 1) / LV : 1;     // units per column
+  // units in n analyses, and the position of a unit
+  auto units = [&](long long n) { return LV > 1 ? n / p.nzc * upc : n; };
+  auto at_unit = [&](long long u) { return LV > 1 ? u / upc * p.nzc + u % upc * LV : u; };
   const int wave = threadIdx.x >> 6;
   const int apb = (blockDim.x >> 6) / WPA;
   if constexpr (SCHED == 0) {
     const long long li = (long long)xcd_block(p.n_blocks) * apb + wave / WPA;
-    if (li >= p.n_an) return;
-    body(analysis_at(p, li));
+    if (li >= units(p.n_an)) return;
+    body(analysis_at(p, at_unit(li)));
     return;
   }
   constexpr bool timing = SCHED == 2 || SCHED == 4;
   const bool leader = lane == 0 && (WPA == 1 || wave == 0);
-  const long long lo = p.seg_off[p.seg_lo], hi = p.seg_off[p.seg_hi], len = hi - lo;
+  const long long lo = p.seg_off[p.seg_lo], len = p.seg_off[p.seg_hi] - lo;
   auto bucket_of_pos = [&](long long pos) {
     int j = p.seg_lo;
     while (j + 1 < p.seg_hi && pos >= p.seg_off[j + 1]) ++j;
@@ -471,10 +478,10 @@ __device__ __forceinline__ void for_analyses(const ProdParams& p, int lane, Body
     long long q = (long long)(blockIdx.x >> 3) * apb + wave / WPA;   // index in x's share
     long long pos = -1;
     for (int j = p.seg_lo; j < p.seg_hi; ++j) {
-      const long long b0 = p.seg_off[j], nb = p.seg_off[j + 1] - b0;
-      const long long e0 = b0 + nb * x / 8, e1 = b0 + nb * (x + 1) / 8;
+      const long long b0 = p.seg_off[j], nb = units(p.seg_off[j + 1] - b0);
+      const long long e0 = nb * x / 8, e1 = nb * (x + 1) / 8;
       if (q < e1 - e0) {
-        pos = e0 + q;
+        pos = b0 + at_unit(e0 + q);
         break;
       }
       q -= e1 - e0;
@@ -512,10 +519,11 @@ __device__ __forceinline__ void for_analyses(const ProdParams& p, int lane, Body
       v = __builtin_amdgcn_readfirstlane(s_next);
       __syncthreads();
     }
-    const long long c0 = kQueueSplit ? lo + len * vx / 8 : lo;
-    const long long c1 = kQueueSplit ? lo + len * (vx + 1) / 8 : hi;
-    const long long pos = c0 + v;
-    if (pos >= c1) {
+    const long long nu = units(len);
+    const long long c0 = kQueueSplit ? nu * vx / 8 : 0;
+    const long long c1 = kQueueSplit ? nu * (vx + 1) / 8 : nu;
+    const long long pos = lo + at_unit(c0 + v);
+    if (c0 + v >= c1) {
       if (++tried == 8) break;
       vx = (vx + 1) & 7;
       continue;
@@ -828,6 +836,268 @@ __global__ __launch_bounds__(256) void k_products_f32(ProdParams p) {
       if (wsub == 1) products_f32_wave<KP, 1, PPW, PW>(p, a, ah, vc, r0, r1, lane);
       if (wsub == 2) products_f32_wave<KP, 2, PPW, PW>(p, a, ah, vc, r0, r1, lane);
       if (wsub == 3) products_f32_wave<KP, 3, PPW, PW>(p, a, ah, vc, r0, r1, lane);
+    }
+  });
+}
+
+// The level loop's products (FP64 or FP32 MFMA, REAL): one wavefront (KP =
+// 128: four sharing the tiles) runs LV consecutive levels of a column.  They
+// share the column's row list, so a row's Yb is gathered once for all of them,
+// and its weights, which differ by the vertical factor only, are formed 64
+// rows at a time, one row per lane, and read back from LDS (formed beside the
+// MFMAs they took every lane of a quarter through the same row's division and
+// polynomial, 16 times over, and bound the kernel).  The MFMAs and the sums of
+// b run in the order of the per-analysis kernels: the same bits.
+// 360x180x32, k = 32, 3.2 G rows: 138 -> 55 ms (MFMA issue is 32 of it).
+template <class REAL> struct LevelReal;
+template <> struct LevelReal<double> {
+  using acc = d4;
+  static __device__ __forceinline__ acc mma(double x, double y, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ double fma_(double x, double y, double c) { return fma(x, y, c); }
+  static __device__ __forceinline__ const double* yb(const ProdParams& p) { return p.yb64; }
+  static __device__ __forceinline__ int out_row(int q, int r) { return q + 4 * r; }
+};
+template <> struct LevelReal<float> {
+  using acc = f4;
+  static __device__ __forceinline__ acc mma(float x, float y, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ float fma_(float x, float y, float c) { return fmaf(x, y, c); }
+  static __device__ __forceinline__ const float* yb(const ProdParams& p) { return p.yb32; }
+  static __device__ __forceinline__ int out_row(int q, int r) { return 4 * q + r; }
+};
+
+// levels per visit: the accumulators of LV levels (tiles x 4 registers, 8 for
+// FP64) beside the loads in flight against wavefronts per SIMD (k = 32 FP32:
+// 2 levels 55 ms, 4 64 ms, 8 80 ms)
+template <int KP, class REAL>
+constexpr int level_count() {
+  return KP == 32 || sizeof(REAL) == 4 ? 2 : 1;
+}
+
+template <int LV, class REAL>
+struct LevelLds {
+  int row[2][64];                    // FP32: byte offset of the row in Yb
+  REAL w[LV][64][2];                 // {w, w d} per level and row
+};
+
+template <int KP, int WS, int PPW, int LV, class REAL>
+__device__ __forceinline__ void products_levels_wave(const ProdParams& p, long long a, int nlv,
+                                                     const double (&vc)[LV], long long r0,
+                                                     long long r1, int lane,
+                                                     LevelLds<LV, REAL>& sh) {
+  using LR = LevelReal<REAL>;
+  using acc_t = typename LR::acc;
+  constexpr int T = KP / 16;
+  using PT = PairTable<T>;
+  constexpr int P0 = WS * PPW;
+  constexpr int P1 = (P0 + PPW < PT::N) ? P0 + PPW : PT::N;
+  constexpr int NP = P1 - P0;
+  const int i16 = lane & 15, q = lane >> 4;
+  acc_t acc[LV][NP];
+  REAL bacc[LV][T];
+#pragma unroll
+  for (int v = 0; v < LV; ++v) {
+#pragma unroll
+    for (int x = 0; x < NP; ++x) acc[v][x] = acc_t{0, 0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < T; ++t) bacc[v][t] = 0;
+  }
+  const int n = (int)(r1 - r0);
+  const REAL* __restrict__ yb = LR::yb(p);
+  // lane's row of the 64-row block at `base` (positions past the end take the
+  // list's last row and weight 0)
+  struct Row { int row; double gc, rinv, vco, dep; bool in; };
+  auto load_list = [&](int base, Row& w) {
+    const int rl = base + lane;
+    w.in = rl < n;
+    const int rc = w.in ? rl : n - 1;
+    w.row = p.row_idx[r0 + rc];
+    w.gc = p.row_gc[r0 + rc];
+  };
+  auto load_obs = [&](Row& w) {
+    w.rinv = (double)p.rinv32[w.row];
+    w.vco = p.vco[w.row];
+    w.dep = p.dep[w.row];
+  };
+  auto put_weights = [&](const Row& w) {
+#pragma unroll
+    for (int v = 0; v < LV; ++v) {
+#pragma clang fp contract(off)
+      // row_weight and the products' w d
+      double x = w.rinv * w.gc;
+      x = x * gc_weight(fabs(vc[v] - w.vco) / p.vert_dist, p.gc_filter_vertical);
+      const double xd = x * w.dep;
+      sh.w[v][lane][0] = w.in ? (REAL)x : (REAL)0;
+      sh.w[v][lane][1] = w.in ? (REAL)xd : (REAL)0;
+    }
+  };
+  // FP32 rows at 32-bit byte offsets (below kYbOffsetLimit)
+  unsigned mo[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) mo[t] = sizeof(REAL) * min(16 * t + i16, p.k - 1);
+  const int unit = sizeof(REAL) == 4 ? 4 * p.k : 1;
+  auto load_y = [&](int buf, int at, REAL (&y)[T]) {
+    const int ro = sh.row[buf][at];
+    const char* yr = reinterpret_cast<const char*>(yb) +
+                     (sizeof(REAL) == 4 ? 0 : (long long)ro * p.k * (long long)sizeof(REAL));
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const REAL yl = *reinterpret_cast<const REAL*>(yr + (sizeof(REAL) == 4 ? ro + mo[t] : mo[t]));
+      y[t] = 16 * t + i16 < p.k ? yl : (REAL)0;
+    }
+  };
+  // FP32 sums of long lists go to FP64 every kFlushRows rows, as in the
+  // per-analysis kernel
+  double* A = p.A + (a - p.a0) * (long long)KP * KP;
+  constexpr long long KK = (long long)KP * KP;
+  const bool chunked = sizeof(REAL) == 4 && n > kFlushMinRows;
+  bool flushed = false;
+  double bsum[LV][T];
+#pragma unroll
+  for (int v = 0; v < LV; ++v)
+#pragma unroll
+    for (int t = 0; t < T; ++t) bsum[v][t] = 0.0;
+
+  constexpr int G = 2;               // groups of 4 rows gathered ahead of the MFMAs
+  if (n > 0) {
+    Row cur, nxt;
+    load_list(0, cur);
+    load_obs(cur);
+    sh.row[0][lane] = cur.row * unit;
+    put_weights(cur);
+    __builtin_amdgcn_wave_barrier();
+    REAL yn[G][T];
+#pragma unroll
+    for (int g = 0; g < G; ++g) load_y(0, 4 * g + q, yn[g]);
+    int buf = 0;
+    for (int base = 0; base < n; base += 64, buf ^= 1) {
+      if constexpr (sizeof(REAL) == 4) {
+        if (chunked && base > 0 && base % kFlushRows == 0) {
+#pragma unroll
+          for (int v = 0; v < LV; ++v) {
+            if (v >= nlv) continue;
+#pragma unroll
+            for (int x = 0; x < NP; ++x) {
+              const int I = PT::I(P0 + x), J = PT::J(P0 + x);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                double* e = A + v * KK + (long long)(16 * J + i16) * KP + 16 * I + LR::out_row(q, r);
+                *e = (flushed ? *e : 0.0) + (double)acc[v][x][r];
+              }
+              acc[v][x] = acc_t{0, 0, 0, 0};
+            }
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+              bsum[v][t] += (double)bacc[v][t];
+              bacc[v][t] = 0;
+            }
+          }
+          flushed = true;
+        }
+      }
+      // the next block's list entries now, its obs values and row numbers
+      // after half of this block, its weights after all of it
+      const bool more = base + 64 < n;
+      load_list(more ? base + 64 : base, nxt);
+      const int ng = min(16, (n - base + 3) / 4);
+#pragma unroll 1
+      for (int h = 0; h < 2; ++h) {
+        if (h == 1) {
+          load_obs(nxt);
+          sh.row[buf ^ 1][lane] = nxt.row * unit;
+          __builtin_amdgcn_wave_barrier();
+        }
+#pragma unroll 1
+        for (int g0 = 8 * h; g0 < 8 * h + 8 && g0 < ng; g0 += G) {
+          REAL y[G][T];
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int t = 0; t < T; ++t) y[g][t] = yn[g][t];
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            const int gn = g0 + G + g;
+            load_y(gn < 16 ? buf : buf ^ 1, 4 * (gn & 15) + q, yn[g]);
+          }
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+#pragma unroll
+            for (int v = 0; v < LV; ++v) {
+              const REAL w = sh.w[v][4 * (g0 + g) + q][0], wd = sh.w[v][4 * (g0 + g) + q][1];
+#pragma unroll
+              for (int x = 0; x < NP; ++x) {
+                const int I = PT::I(P0 + x), J = PT::J(P0 + x);
+                acc[v][x] = LR::mma(y[g][I], w * y[g][J], acc[v][x]);
+              }
+              if (WS == 0) {
+#pragma unroll
+                for (int t = 0; t < T; ++t) bacc[v][t] = LR::fma_(wd, y[g][t], bacc[v][t]);
+              }
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      put_weights(nxt);
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < LV; ++v) {
+    if (v >= nlv) continue;
+#pragma unroll
+    for (int x = 0; x < NP; ++x) {
+      const int I = PT::I(P0 + x), J = PT::J(P0 + x);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * I + LR::out_row(q, r), col = 16 * J + i16;
+        const double e = (flushed ? A[v * KK + (long long)col * KP + row] : 0.0) + (double)acc[v][x][r];
+        A[v * KK + (long long)col * KP + row] = e;
+        if (I != J) A[v * KK + (long long)row * KP + col] = e;
+      }
+    }
+    if (WS == 0) {
+      double* b = p.b + (a - p.a0 + v) * KP;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        double e = bsum[v][t] + (double)bacc[v][t];
+        e += __shfl_xor(e, 16, 64);
+        e += __shfl_xor(e, 32, 64);
+        if (q == 0) b[16 * t + i16] = e;
+      }
+    }
+  }
+}
+
+template <int KP, class REAL, int SCHED>
+__global__ __launch_bounds__(256) void k_products_levels(ProdParams p) {
+  constexpr int T = KP / 16;
+  constexpr int NPAIR = T * (T + 1) / 2;
+  constexpr int WPA = (NPAIR + 9) / 10;
+  constexpr int PPW = (NPAIR + WPA - 1) / WPA;
+  constexpr int LV = level_count<KP, REAL>();
+  __shared__ LevelLds<LV, REAL> sh[WPA];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wsub = wave % WPA;
+  for_analyses<WPA, SCHED, LV>(p, lane, [&](long long li) {
+    const long long a = p.a0 + li;
+    const int ah = (int)(a / p.nzc), kc = (int)(a % p.nzc);
+    // row lists past the list buffer's capacity are cut at it, as in
+    // k_products_f64
+    const long long r0 = min(p.row_off[ah - p.h0], p.row_cap);
+    const long long r1 = min(p.row_off[ah - p.h0 + 1], p.row_cap);
+    const int nlv = min(LV, p.nzc - kc);
+    double vc[LV];
+#pragma unroll
+    for (int v = 0; v < LV; ++v) vc[v] = chunk_vcoord(p, ah, min(kc + v, p.nzc - 1));
+    if (wsub == 0) products_levels_wave<KP, 0, PPW, LV, REAL>(p, a, nlv, vc, r0, r1, lane, sh[0]);
+    if constexpr (WPA > 1) {
+      if (wsub == 1) products_levels_wave<KP, 1, PPW, LV, REAL>(p, a, nlv, vc, r0, r1, lane, sh[1]);
+      if (wsub == 2) products_levels_wave<KP, 2, PPW, LV, REAL>(p, a, nlv, vc, r0, r1, lane, sh[2]);
+      if (wsub == 3) products_levels_wave<KP, 3, PPW, LV, REAL>(p, a, nlv, vc, r0, r1, lane, sh[3]);
     }
   });
 }
@@ -1997,9 +2267,11 @@ static int resident_blocks(const void* f, int threads, std::atomic<int>& cache) 
 // One workgroup per analysis: its wavefronts (one, or four sharing the
 // analysis) start and retire together, so no wavefront waits on another
 // analysis of its workgroup.
+// lv: levels of a column that a visit covers (level loop).
 template <class K>
 static hipError_t launch_prod(hipStream_t st, const ProdParams& p, K* kern, long long blocks,
-                              std::atomic<int>& cache, int wpa, long long* capacity) {
+                              std::atomic<int>& cache, int wpa, long long* capacity, int lv = 1) {
+  if (lv > 1) blocks = blocks / p.nzc * ((p.nzc + lv - 1) / lv);
   ProdParams q = p;
   unsigned grid;
   constexpr int apb = 1;
@@ -2014,7 +2286,7 @@ static hipError_t launch_prod(hipStream_t st, const ProdParams& p, K* kern, long
   } else if (q.order) {
     // an XCD's share is an eighth of each bucket, rounded: at most
     // n / 8 + kBuckets analyses
-    const long long per_xcd = ((q.n_an + 7) / 8 + kBuckets + apb - 1) / apb;
+    const long long per_xcd = ((blocks + 7) / 8 + kBuckets + apb - 1) / apb;
     grid = (unsigned)(8 * per_xcd);
     q.n_blocks = (int)grid;
   } else {
@@ -2036,8 +2308,15 @@ static hipError_t launch_products_sched(hipStream_t st, const ProdParams& p, int
   // PW: the row lists carry the weights w and w d (horizontal loop), so the
   // products read them instead of forming them per row; straight-line code
   // lets a group's loads be in flight together
-  static std::atomic<int> c64[2], c32[2], c16a[2], c16b[2];
+  static std::atomic<int> c64[2], c32[2], c16a[2], c16b[2], cl[2];
   const int w = p.pre_weighted ? 1 : 0;
+  // the level loop: the weights are formed per row and level
+  if (p.vertical && !w && precision == 0)
+    return launch_prod(st, p, k_products_levels<KP, double, SCHED>, blocks, cl[0], WPA, capacity,
+                       level_count<KP, double>());
+  if (p.vertical && !w && precision == 1)
+    return launch_prod(st, p, k_products_levels<KP, float, SCHED>, blocks, cl[1], WPA, capacity,
+                       level_count<KP, float>());
   if (precision == 0)
     return w ? launch_prod(st, p, k_products_f64<KP, SCHED, true>, blocks, c64[1], WPA, capacity)
              : launch_prod(st, p, k_products_f64<KP, SCHED, false>, blocks, c64[0], WPA, capacity);

@@ -1,0 +1,56 @@
+"""GPU tests of the level loop's products (several levels of a column per
+wavefront, row weights 64 rows at a time): ensemble widths of each kernel,
+odd level counts, row lists from empty to several blocks of 64 with every
+remainder, in the bucket order and in column order, against the oracle.
+
+FP64 at the repository's 1e-10; FP32 products at its increment bound, 1e-5
+RMS of the FP64 increment per call."""
+import copy
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    torch.cuda.set_device(0)
+
+
+@pytest.mark.parametrize("schedule", [1, 0])
+@pytest.mark.parametrize("k,nz,cube_nz,n_obs", [
+    (8, 5, 1, 30), (31, 4, 1, 400), (32, 7, 2, 2500), (33, 3, 1, 400), (64, 5, 2, 900),
+    (65, 3, 1, 300), (128, 2, 1, 700), (20, 5, 3, 9000)])
+def test_level_products(k, nz, cube_nz, n_obs, schedule):
+    import orc
+    from dida_letkf import engine, synth
+    inst = synth.generate("c1", seed=k + n_obs, k=k, nlat=6, nlon=11, nz=nz, n_obs=n_obs,
+                          local_dist=700.0)
+    inst.cfg.vert_dist = 1.1
+    inst.cfg.cube_nz = cube_nz
+    ref = orc.letkf_compute(inst, want_trans=True)
+    full = ref["xa"] + ref["axa"][..., None]
+    inc = np.sqrt(np.mean((full - inst.xb - inst.axb[..., None]) ** 2))
+    for prec in (0, 1):
+        cfg = copy.copy(inst.cfg)
+        cfg.precision = prec
+        with engine.LetkfEngine(cfg, keep_transforms=True) as eng:
+            eng.set_option(engine.OPT_SCHEDULE, schedule)
+            eng.set_grid(inst.grid_lat, inst.grid_lon)
+            eng.set_obs(inst.obs)
+            xa, axa, rc = eng.letkf_compute(inst.xb, inst.axb)
+            _, _, nobsl = eng.get_transforms()
+        assert rc == 0 and np.array_equal(nobsl, ref["nobsl"])
+        got = xa + axa[..., None]
+        if prec == 0:
+            err = np.abs(got - full).max() / np.abs(full).max()
+            print(k, nz, n_obs, "p", nobsl.min(), nobsl.max(), "fp64", err, flush=True)
+            assert err < 1e-10
+        else:
+            err = np.sqrt(np.mean((got - full) ** 2)) / inc
+            print(k, nz, n_obs, "fp32 increment", err, flush=True)
+            assert err < 1e-5
