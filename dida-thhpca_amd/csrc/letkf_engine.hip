@@ -157,6 +157,20 @@ __global__ void k_f64_to_f32(long long n, const double* __restrict__ in, float* 
   if (i < n) out[i] = (float)in[i];
 }
 
+// *bad = 1 where a value the products read is not finite (Yb in their precision)
+template <class REAL>
+__global__ void k_obs_bad(long long ny, const REAL* __restrict__ yb, long long n_rows,
+                          const double* __restrict__ dep, const float* __restrict__ rinv,
+                          int* __restrict__ bad) {
+  const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long step = (long long)gridDim.x * blockDim.x;
+  bool b = false;
+  for (long long i = i0; i < ny; i += step) b = b || !__builtin_isfinite(yb[i]);
+  for (long long i = i0; i < n_rows; i += step)
+    b = b || !__builtin_isfinite(dep[i]) || !__builtin_isfinite(rinv[i]);
+  if (b) *bad = 1;                   // every writer stores the same value
+}
+
 // out[i] = i for i < n, then 0 for the list padding up to n + pad
 __global__ void k_iota(long long n, long long pad, int* __restrict__ out) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -541,7 +555,7 @@ struct dida_letkf_handle {
   double bdeg_lat = 0, bdeg_lon = 0, theta_deg = 0;
   DevBuf key_in, key_out, val_in, val_out, hist, bin_start, sort_tmp;
   DevBuf s_cos, s_sin, s_lonr, s_cosl, s_sinl, s_row0, s_nrow;
-  DevBuf yb32, rinv32;
+  DevBuf yb32, rinv32, obs_bad;
   DevBuf d_hyai, d_hybi;
   DevBuf row_site, nobsl_dev;         // tile-mode selection and row counts
   // work
@@ -714,7 +728,7 @@ int dida_letkf_destroy(dida_letkf_handle* h) {
                     &h->o_dep, &h->o_rinv64, &h->o_vco, &h->key_in, &h->key_out, &h->val_in,
                     &h->val_out, &h->hist, &h->bin_start, &h->sort_tmp, &h->s_cos, &h->s_sin,
                     &h->s_lonr, &h->s_cosl, &h->s_sinl, &h->s_row0, &h->s_nrow, &h->yb32,
-                    &h->rinv32, &h->d_hyai,
+                    &h->rinv32, &h->obs_bad, &h->d_hyai,
                     &h->d_hybi, &h->cnt, &h->off, &h->scan_tmp, &h->row_idx, &h->row_gc,
                     &h->row_site, &h->nobsl_dev, &h->row_wd,
                     &h->Abuf, &h->bbuf, &h->status, &h->trans, &h->wout, &h->x_xb, &h->x_axb,
@@ -858,6 +872,19 @@ static int build_obs_index(dida_letkf_handle* h, int n_sites, const double* lat,
     if (ny > 0)
       hipLaunchKernelGGL(k_f64_to_f32, dim3((unsigned)((ny + 255) / 256)), dim3(256), 0, st, ny,
                          yb, h->yb32.as<float>());
+  }
+  // the level loop leaves out rows of vertical weight 0 where all is finite
+  if (c.vert_dist > 0.0) {
+    RC_TRY(h->obs_bad.ensure(sizeof(int)));
+    HIP_TRY(launch_zero_ints(st, h->obs_bad.as<int>(), 1));
+    const long long ny = (long long)n_rows * c.k;
+    const dim3 grid((unsigned)std::min<long long>((ny + 1023) / 1024, 2048));
+    if (ny > 0 && c.precision == DIDA_PREC_FP64)
+      hipLaunchKernelGGL(k_obs_bad<double>, grid, dim3(256), 0, st, ny, yb, (long long)n_rows, dep,
+                         h->rinv32.as<float>(), h->obs_bad.as<int>());
+    else if (ny > 0)
+      hipLaunchKernelGGL(k_obs_bad<float>, grid, dim3(256), 0, st, ny, h->yb32.as<float>(),
+                         (long long)n_rows, dep, h->rinv32.as<float>(), h->obs_bad.as<int>());
   }
   HIP_TRY(hipGetLastError());
   h->have_obs = true;
@@ -1292,6 +1319,7 @@ static int enqueue_call(dida_letkf_handle* h, const StateArgs& sa, bool timed, i
     pp.dep = h->o_dep.as<double>();
     pp.rinv32 = h->rinv32.as<float>();
     pp.vco = h->o_vco.as<double>();
+    pp.obs_bad = h->obs_bad.as<int>();
     pp.a0 = h0 * h->nzc;
     pp.n_an = (h1 - h0) * h->nzc;
     pp.groups = 1;
@@ -1571,7 +1599,8 @@ static std::vector<uintptr_t> graph_key(const dida_letkf_handle* h, const StateA
   // enough, so a new cycle's obs replay the same graph)
   for (const DevBuf* b : {&h->glat, &h->glon, &h->o_yb64, &h->o_dep, &h->o_vco, &h->bin_start,
                           &h->s_cos, &h->s_sin, &h->s_lonr, &h->s_cosl, &h->s_sinl, &h->s_row0,
-                          &h->s_nrow, &h->yb32, &h->rinv32, &h->d_hyai, &h->d_hybi})
+                          &h->s_nrow, &h->yb32, &h->rinv32, &h->obs_bad, &h->d_hyai,
+                          &h->d_hybi})
     put(b->p);
   k.push_back((uintptr_t)h->row_cap);
   k.push_back((uintptr_t)h->opt_schedule);

@@ -114,6 +114,7 @@ struct ProdParams {
   const double* dep;
   const float* rinv32;
   const double* vco;
+  const int* obs_bad;        // level loop: 1 if a Yb, d or R^-1 of the obs set is not finite
   long long a0, n_an;        // analyses [a0, a0 + n_an)
   int h0;
   double* A;                 // batch-local, kp*kp per analysis

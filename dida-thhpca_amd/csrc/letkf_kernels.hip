@@ -847,8 +847,17 @@ __global__ __launch_bounds__(256) void k_products_f32(ProdParams p) {
 // rows at a time, one row per lane, and read back from LDS (formed beside the
 // MFMAs they took every lane of a quarter through the same row's division and
 // polynomial, 16 times over, and bound the kernel).  The MFMAs and the sums of
-// b run in the order of the per-analysis kernels: the same bits.
-// 360x180x32, k = 32, 3.2 G rows: 138 -> 55 ms (MFMA issue is 32 of it).
+// b run in the order of the list.
+//
+// Most rows of a column lie outside the vertical support of a level (74% of
+// them at 32 levels and a support of +-4), where their weight is exactly 0.
+// A first look at 64 rows' vertical coordinate keeps the rows that may carry
+// weight at one of the wavefront's levels in a ring, in list order, and the
+// weights, the gathers and the MFMAs take blocks of 64 kept rows.  A row with
+// weight 0 adds exact zeros unless its Yb, d or R^-1 is not finite: obs sets
+// that hold such a value (obs_bad) keep every row.
+// 360x180x32, k = 32, 3.2 G rows, FP32: 138 ms with weights beside the MFMAs,
+// 55 ms with blocks of 64 unfiltered rows, 22 ms now (cycle 108 -> 77 ms).
 template <class REAL> struct LevelReal;
 template <> struct LevelReal<double> {
   using acc = d4;
@@ -879,6 +888,7 @@ constexpr int level_count() {
 
 template <int LV, class REAL>
 struct LevelLds {
+  int pend_row[128], pend_pos[128];  // ring of kept rows: row and list position
   int row[2][64];                    // FP32: byte offset of the row in Yb
   REAL w[LV][64][2];                 // {w, w d} per level and row
 };
@@ -907,15 +917,55 @@ __device__ __forceinline__ void products_levels_wave(const ProdParams& p, long l
   }
   const int n = (int)(r1 - r0);
   const REAL* __restrict__ yb = LR::yb(p);
-  // lane's row of the 64-row block at `base` (positions past the end take the
-  // list's last row and weight 0)
+  // rows that may carry weight, found 64 list positions at a time: `scan` is
+  // the next position, its rows (fr0) and their coordinate (fv0) are in
+  // flight, and so are the rows after them (fr1).  The bound is a little above
+  // 2 vert_dist, so a row it drops has |vc - vco| / vert_dist > 2 however the
+  // division rounds; a NaN coordinate is kept
+  const double lim = 2.0 * p.vert_dist * (1.0 + 1e-12);
+  const bool keep_all = *p.obs_bad != 0;
+  const unsigned long long below = (1ull << lane) - 1;
+  int scan = 0, head = 0, pend = 0, fr0 = 0, fr1 = 0;
+  double fv0 = 0.0;
+  if (n > 0) {
+    fr0 = p.row_idx[r0 + min(lane, n - 1)];
+    fr1 = p.row_idx[r0 + min(64 + lane, n - 1)];
+    fv0 = p.vco[fr0];
+  }
+  auto refill = [&]() {              // at most 63 + 64 rows pend
+    while (pend < 64 && scan < n) {
+      bool keep = keep_all;
+#pragma unroll
+      for (int v = 0; v < LV; ++v) keep = keep || !(fabs(vc[v] - fv0) > lim);
+      keep = keep && scan + lane < n;
+      const unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
+      if (keep) {
+        const int s = (head + pend + __popcll(m & below)) & 127;
+        sh.pend_row[s] = fr0;
+        sh.pend_pos[s] = scan + lane;
+      }
+      pend += __popcll(m);
+      scan += 64;
+      fr0 = fr1;
+      fv0 = p.vco[fr0];
+      fr1 = p.row_idx[r0 + min(scan + 64 + lane, n - 1)];
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  // lane's row of the next 64 pending rows (lanes past their end take the
+  // last one and weight 0); returns their number, 0 leaves the row as it is
   struct Row { int row; double gc, rinv, vco, dep; bool in; };
-  auto load_list = [&](int base, Row& w) {
-    const int rl = base + lane;
-    w.in = rl < n;
-    const int rc = w.in ? rl : n - 1;
-    w.row = p.row_idx[r0 + rc];
-    w.gc = p.row_gc[r0 + rc];
+  auto take = [&](Row& w) -> int {
+    const int c = min(pend, 64);
+    if (c > 0) {
+      const int s = (head + min(lane, c - 1)) & 127;
+      w.row = sh.pend_row[s];
+      w.gc = p.row_gc[r0 + sh.pend_pos[s]];
+      head += c;
+      pend -= c;
+    }
+    w.in = lane < c;
+    return c;
   };
   auto load_obs = [&](Row& w) {
     w.rinv = (double)p.rinv32[w.row];
@@ -962,18 +1012,19 @@ __device__ __forceinline__ void products_levels_wave(const ProdParams& p, long l
     for (int t = 0; t < T; ++t) bsum[v][t] = 0.0;
 
   constexpr int G = 2;               // groups of 4 rows gathered ahead of the MFMAs
-  if (n > 0) {
-    Row cur, nxt;
-    load_list(0, cur);
-    load_obs(cur);
-    sh.row[0][lane] = cur.row * unit;
-    put_weights(cur);
+  refill();
+  Row blk;
+  int nb = take(blk);
+  if (nb > 0) {
+    load_obs(blk);
+    sh.row[0][lane] = blk.row * unit;
+    put_weights(blk);
     __builtin_amdgcn_wave_barrier();
     REAL yn[G][T];
 #pragma unroll
     for (int g = 0; g < G; ++g) load_y(0, 4 * g + q, yn[g]);
     int buf = 0;
-    for (int base = 0; base < n; base += 64, buf ^= 1) {
+    for (int base = 0; nb > 0; base += 64, buf ^= 1) {
       if constexpr (sizeof(REAL) == 4) {
         if (chunked && base > 0 && base % kFlushRows == 0) {
 #pragma unroll
@@ -999,15 +1050,16 @@ __device__ __forceinline__ void products_levels_wave(const ProdParams& p, long l
         }
       }
       // the next block's list entries now, its obs values and row numbers
-      // after half of this block, its weights after all of it
-      const bool more = base + 64 < n;
-      load_list(more ? base + 64 : base, nxt);
-      const int ng = min(16, (n - base + 3) / 4);
+      // after half of this block, its weights after all of it (after the last
+      // block its rows again, with weight 0)
+      const int ng = (nb + 3) / 4;
+      refill();
+      nb = take(blk);
 #pragma unroll 1
       for (int h = 0; h < 2; ++h) {
         if (h == 1) {
-          load_obs(nxt);
-          sh.row[buf ^ 1][lane] = nxt.row * unit;
+          load_obs(blk);
+          sh.row[buf ^ 1][lane] = blk.row * unit;
           __builtin_amdgcn_wave_barrier();
         }
 #pragma unroll 1
@@ -1041,7 +1093,7 @@ __device__ __forceinline__ void products_levels_wave(const ProdParams& p, long l
         }
       }
       __builtin_amdgcn_wave_barrier();
-      put_weights(nxt);
+      put_weights(blk);
       __builtin_amdgcn_wave_barrier();
     }
   }
