@@ -1515,8 +1515,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
         for (int J = 0; J < 2; ++J)
 #pragma unroll
-          for (int rr = 0; rr < 4; ++rr)
-            refl[tile_off<KMAX>(4 * pass + I, 2 * wv + J, rr, lane)] = acc[I][J][rr];
+          for (int rr = 0; rr < 4; ++rr) {
+            // in the precision of the state, as k_vec leaves it
+            const int o = tile_off<KMAX>(4 * pass + I, 2 * wv + J, rr, lane);
+            if (p.state_f32) reinterpret_cast<float*>(refl)[o] = (float)acc[I][J][rr];
+            else refl[o] = acc[I][J][rr];
+          }
     }
   }
   // every thread scans overline_w in LDS, so the decision is uniform
@@ -1531,16 +1535,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   if (p.w_out && h == 0 && in_r) p.w_out[a * (long long)k + r] = sw[r];
 }
 
-// Xa = Xb trans for k = 65..128: wave w produces members 32w .. 32w+31 from the
-// trans tiles J in {2w, 2w+1}; 16 state vectors per MFMA group.  TS and EPI
-// as k_update.
+// Xa = Xb trans for k = 65..128: wave w produces members 32w .. 32w+31, its
+// trans columns (128 x 32) in registers; all four take the same groups of 16
+// state vectors.  TS and EPI as k_update.
+//
+// The bound is the state and trans in HBM (10.7 GB for the FP32 state of
+// 64,800 columns of 97 vectors at k = 128) and the f32 MFMAs beside it.  A
+// operands come straight from the state: the MFMA reduction index is permuted
+// so that a lane's operands are 16-byte pieces of its vector (step s, lane
+// quarter q carry member 4 VEC (s / VEC) + VEC q + s mod VEC, so one load
+// instruction covers 64 contiguous bytes of each of 16 vectors), the next
+// group's as soon as the MFMAs have consumed this one's; LDS only carries the
+// wavefronts' shares of the means, one barrier a group.  (Staged through LDS
+// between two barriers a group, with no load in flight across them, and sums
+// by shuffles, 10.7 ms there; now 4.3 ms.)
 template <class TS, int EPI>
-__global__ __launch_bounds__(256) void k_update128(EigParams p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void k_update128(EigParams p) {
   using ST = StateT<TS>;
   using acc_t = typename ST::acc;
-  constexpr int KMAX = 128, LDV = KMAX + 1, NT = 256;
-  __shared__ TS sV[16 * LDV];
-  __shared__ double spart[3][4][16];
+  constexpr int KMAX = 128, S = KMAX / 4;
+  constexpr int VEC = 16 / sizeof(TS);       // members per 16-byte load
+  // shares of the sums of a group's 16 vectors: of the members (a buffer for
+  // each of two groups in turn), and with EPI of the two spreads
+  __shared__ double spart[2][4][16];
+  __shared__ double sspr[EPI ? 2 : 1][4][16];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
   long long a, ai, ar;
@@ -1555,153 +1574,192 @@ __global__ __launch_bounds__(256) void k_update128(EigParams p) {
   // q + 4 rr for f64 16x16x4, 4 q + rr for f32 16x16x4
   constexpr bool F32 = sizeof(TS) == 4;
   auto out_row = [q](int rr) { return F32 ? 4 * q + rr : q + 4 * rr; };
+  auto member = [q](int s) { return 4 * VEC * (s / VEC) + VEC * q + s % VEC; };
   const TS* __restrict__ xb = ST::xb(p);
-  const double* __restrict__ tb = p.refl + ai * (long long)kp * kp;
-  TS bop[8][2][4];
+  // trans tiles from the transform, in the state's precision
+  const TS* __restrict__ tb =
+      reinterpret_cast<const TS*>(p.refl + ai * (long long)kp * kp);
+  // tile_off of member(s)'s row, split in the lane's part and a constant
+  const TS* __restrict__ tl =
+      tb + tile_off<KMAX>(0, 2 * wv, F32 ? q : q >> 1, (F32 ? 0 : 32 * (q & 1)) + i16);
+  TS bop[S][2];
 #pragma unroll
-  for (int I = 0; I < 8; ++I)
+  for (int s = 0; s < S; ++s) {
 #pragma unroll
     for (int J = 0; J < 2; ++J)
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) bop[I][J][rr] = (TS)tb[tile_off<KMAX>(I, 2 * wv + J, rr, lane)];
+      bop[s][J] = tl[tile_off<KMAX>(s >> 2, J, F32 ? 0 : s & 2, 16 * (F32 ? s & 3 : s & 1))];
+    if (s % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+  }
 
   const AnRows R = an_rows(p, a);
   const int sj = R.sj, ej = R.ej, si = R.si, ei = R.ei, sk = R.sk, ek = R.ek;
   const long long lat_ext = R.lat_ext;
-  int rs[kMaxVars], rl[kMaxVars];
-  int nrun = 0, nvec = 0;
-  if (!p.vertical) {
-    rs[0] = 0; rl[0] = p.n; nrun = 1;
-  } else {
-    for (int vv = 0; vv < p.n_var; ++vv) {
-      const int start = p.var_start[vv] - 1;
-      if (p.var_lev[vv] == 1) {
-        if (ek == p.nz) { rs[nrun] = start; rl[nrun] = 1; ++nrun; }
-      } else {
-        rs[nrun] = start + sk - 1; rl[nrun] = ek - sk + 1; ++nrun;
-      }
-    }
+  // the analysis's state rows, as in k_update
+  auto run_len = [&](int vv) {
+    return p.var_lev[vv] == 1 ? (ek == p.nz ? 1 : 0) : ek - sk + 1;
+  };
+  int nvec = p.n;
+  if (p.vertical) {
+    nvec = 0;
+    for (int vv = 0; vv < p.n_var; ++vv) nvec += run_len(vv);
   }
-  for (int t = 0; t < nrun; ++t) nvec += rl[t];
   auto sidx = [&](int v) {
+    if (v >= nvec) return -1;
+    if (!p.vertical) return v;
     int rem = v;
-    for (int t = 0; t < nrun; ++t) {
-      if (rem < rl[t]) return rs[t] + rem;
-      rem -= rl[t];
+    for (int vv = 0; vv < p.n_var; ++vv) {
+      const int len = run_len(vv);
+      if (rem < len) return p.var_start[vv] - 1 + (p.var_lev[vv] == 1 ? 0 : sk - 1) + rem;
+      rem -= len;
     }
     return -1;
   };
-  for (int lo = si; lo <= ei; ++lo) {
-    for (int la = sj; la <= ej; ++la) {
-      const long long off = ((long long)(lo - 1 + p.halo) * lat_ext + (la - 1 + p.halo)) * p.n;
-      const bool polar = EPI && fabs((double)p.g.glat[la - 1]) > p.polar_lat;
-      for (int v0 = 0; v0 < nvec; v0 += 16) {
-        __syncthreads();
-        for (int e = tid; e < 16 * KMAX; e += NT) {
-          const int u = e / KMAX, m = e % KMAX;
-          const int s_i = (v0 + u < nvec) ? sidx(v0 + u) : -1;
-          sV[u * LDV + m] = (s_i >= 0 && m < k) ? xb[(off + s_i) * k + m] : (TS)0;
+  const int ngrp = (nvec + 15) / 16;
+  const int ncl = ej - sj + 1;
+  const int n_items = (ei - si + 1) * ncl * ngrp;
+  // every vector starts at a 16-byte boundary and ends at a whole piece
+  const bool vec_ld = k % VEC == 0 && (reinterpret_cast<uintptr_t>(xb) & 15) == 0;
+  auto item_off = [&](int it) {
+    const int cl = it / ngrp;
+    const int lo = si + cl / ncl, la = sj + cl % ncl;
+    return ((long long)(lo - 1 + p.halo) * lat_ext + (la - 1 + p.halo)) * p.n;
+  };
+  // steps s0 .. s0 + SA - 1 of item it; FP64's trans fills half of the
+  // registers, so its operands come in two halves, each before its MFMAs
+  constexpr int SA = F32 ? S : S / 2;
+  TS af[SA];
+  auto load_a = [&](int it, auto first) {
+    constexpr int s0 = decltype(first)::value;
+    const int s_a = sidx(16 * (it % ngrp) + i16);
+    const TS* xr = xb + (item_off(it) + (s_a >= 0 ? s_a : 0)) * k;
+    if (vec_ld) {
+#pragma unroll
+      for (int s = 0; s < SA; s += VEC) {
+        // an in-row load and a select: no branch
+        const int m = member(s0 + s);
+        const uint4 t4 = *reinterpret_cast<const uint4*>(xr + (m < k ? m : 0));
+        const TS* tv = reinterpret_cast<const TS*>(&t4);
+#pragma unroll
+        for (int x = 0; x < VEC; ++x) af[s + x] = (s_a >= 0 && m < k) ? tv[x] : (TS)0;
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < SA; ++s) {
+        const int m = member(s0 + s);
+        const TS x = xr[m < k ? m : 0];
+        af[s] = (s_a >= 0 && m < k) ? x : (TS)0;
+        if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // the sum over a row of 16 lanes, in every lane of it
+  auto row_sum = [](double v) {
+    v += dpp_d<0xB1>(v);    // quad_perm [1,0,3,2]
+    v += dpp_d<0x4E>(v);    // quad_perm [2,3,0,1]
+    v += dpp_d<0x141>(v);   // row_half_mirror
+    return v + dpp_d<0x140>(v);   // row_mirror
+  };
+  auto four = [](const double (&x)[4][16], int v) { return (x[0][v] + x[1][v]) + (x[2][v] + x[3][v]); };
+  using First = std::integral_constant<int, 0>;
+  using Second = std::integral_constant<int, S - SA>;
+  if (n_items > 0) load_a(0, First{});
+  for (int it = 0; it < n_items; ++it) {
+    const long long off = item_off(it);
+    const int v0 = 16 * (it % ngrp);
+    double ab4[4];
+    int st4[4];
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+      st4[rr] = sidx(v0 + out_row(rr));
+      ab4[rr] = st4[rr] >= 0 ? p.axb[off + st4[rr]] : 0.0;
+    }
+    acc_t out[2];
+#pragma unroll
+    for (int J = 0; J < 2; ++J) out[J] = acc_t{0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < SA; ++s)
+#pragma unroll
+      for (int J = 0; J < 2; ++J) out[J] = ST::mma(af[s], bop[s][J], out[J]);
+    if constexpr (SA < S) {
+      load_a(it, Second{});
+#pragma unroll
+      for (int s = 0; s < SA; ++s)
+#pragma unroll
+        for (int J = 0; J < 2; ++J) out[J] = ST::mma(af[s], bop[SA + s][J], out[J]);
+    }
+    if (it + 1 < n_items) load_a(it + 1, First{});
+    // lane holds Xa[vector out_row(rr)][member 32w + 16J + i16]
+    double xe[4][2];
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+      double sum = 0.0;
+#pragma unroll
+      for (int J = 0; J < 2; ++J) {
+        const int e = 32 * wv + 16 * J + i16;
+        xe[rr][J] = (e < k) ? (double)out[J][rr] + ab4[rr] : 0.0;
+        sum += xe[rr][J];
+      }
+      sum = row_sum(sum);
+      if (i16 == 0) spart[it & 1][wv][out_row(rr)] = sum;
+    }
+    __syncthreads();
+    if (!EPI) {
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        if (st4[rr] < 0) continue;
+        const double mean = four(spart[it & 1], out_row(rr)) / k;
+        const long long o = off + st4[rr];
+        TS* __restrict__ xa = ST::xa(p);
+#pragma unroll
+        for (int J = 0; J < 2; ++J) {
+          const int e = 32 * wv + 16 * J + i16;
+          if (e < k) xa[o * k + e] = (TS)(xe[rr][J] - mean);
         }
-        __syncthreads();
-        acc_t out[2];
+        if (wv == 0 && i16 == 0) p.axa[o] = mean;
+      }
+    } else {
+      // the caller's epilogue (module_da_parallel.F90:219-261); the spreads'
+      // member sums go through LDS like the mean
+      const int cl = it / ngrp, lo = si + cl / ncl, la = sj + cl % ncl;
+      const bool polar = fabs((double)p.g.glat[la - 1]) > p.polar_lat;
 #pragma unroll
-        for (int J = 0; J < 2; ++J) out[J] = acc_t{0, 0, 0, 0};
+      for (int rr = 0; rr < 4; ++rr) {
+        const int vi = out_row(rr);
+        const double mean = four(spart[it & 1], vi) / k;
+        const long long o = off + (st4[rr] >= 0 ? st4[rr] : 0);
+        double sb = 0.0, sa = 0.0;
 #pragma unroll
-        for (int sK = 0; sK < KMAX / 4; ++sK) {
-          const TS xa_frag = sV[i16 * LDV + 4 * sK + q];
-#pragma unroll
-          for (int J = 0; J < 2; ++J) out[J] = ST::mma(xa_frag, bop[sK >> 2][J][sK & 3], out[J]);
+        for (int J = 0; J < 2; ++J) {
+          const int e = 32 * wv + 16 * J + i16;
+          const bool in = e < k && st4[rr] >= 0;
+          const double xbe = in ? (double)xb[o * k + e] : 0.0;
+          double vv;
+          if (polar) {
+            vv = xbe + ab4[rr];
+            sa += xbe * xbe;
+          } else {
+            vv = p.gamma1 * (ab4[rr] + xbe) + p.gamma2 * (mean + (xe[rr][J] - mean));
+            if (e < k) sa += (vv - mean) * (vv - mean);
+          }
+          sb += xbe * xbe;
+          if (in) p.xa_out[o * k + e] = vv;
         }
-        // lane holds Xa[vector out_row(rr)][member 32w + 16J + i16]
-        double ab4[4], xe[4][2];
+        sb = row_sum(sb);
+        sa = row_sum(sa);
+        if (i16 == 0) {
+          sspr[0][wv][vi] = sb;
+          sspr[EPI ? 1 : 0][wv][vi] = sa;
+        }
+      }
+      __syncthreads();
+      if (wv == 0 && i16 == 0) {
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
-          const int v = v0 + out_row(rr);
-          const int s_i = (v < nvec) ? sidx(v) : -1;
-          ab4[rr] = (s_i >= 0) ? p.axb[off + s_i] : 0.0;
-          double sum = 0.0;
-#pragma unroll
-          for (int J = 0; J < 2; ++J) {
-            const int e = 32 * wv + 16 * J + i16;
-            xe[rr][J] = (e < k) ? (double)out[J][rr] + ab4[rr] : 0.0;
-            sum += xe[rr][J];
-          }
-#pragma unroll
-          for (int o = 1; o < 16; o <<= 1) sum += __shfl_xor(sum, o, 64);
-          if (i16 == 0) spart[0][wv][out_row(rr)] = sum;
-        }
-        __syncthreads();
-        if (!EPI) {
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) {
-            const int v = v0 + out_row(rr);
-            const int s_i = (v < nvec) ? sidx(v) : -1;
-            if (s_i < 0) continue;
-            const int vi = out_row(rr);
-            const double mean =
-                ((spart[0][0][vi] + spart[0][1][vi]) + (spart[0][2][vi] + spart[0][3][vi])) / k;
-            const long long o = off + s_i;
-            TS* __restrict__ xa = ST::xa(p);
-#pragma unroll
-            for (int J = 0; J < 2; ++J) {
-              const int e = 32 * wv + 16 * J + i16;
-              if (e < k) xa[o * k + e] = (TS)(xe[rr][J] - mean);
-            }
-            if (wv == 0 && i16 == 0) p.axa[o] = mean;
-          }
-        } else {
-          // the caller's epilogue (module_da_parallel.F90:219-261); the
-          // spreads' member sums go through LDS like the mean
-          int sidx4[4];
-          double mean4[4];
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) {
-            const int v = v0 + out_row(rr);
-            sidx4[rr] = (v < nvec) ? sidx(v) : -1;
-            const int vi = out_row(rr);
-            mean4[rr] =
-                ((spart[0][0][vi] + spart[0][1][vi]) + (spart[0][2][vi] + spart[0][3][vi])) / k;
-            const long long o = off + (sidx4[rr] >= 0 ? sidx4[rr] : 0);
-            double sb = 0.0, sa = 0.0;
-#pragma unroll
-            for (int J = 0; J < 2; ++J) {
-              const int e = 32 * wv + 16 * J + i16;
-              const bool in = e < k && sidx4[rr] >= 0;
-              const double xbe = in ? (double)xb[o * k + e] : 0.0;
-              double vv;
-              if (polar) {
-                vv = xbe + ab4[rr];
-                sa += xbe * xbe;
-              } else {
-                vv = p.gamma1 * (ab4[rr] + xbe) + p.gamma2 * (mean4[rr] + (xe[rr][J] - mean4[rr]));
-                if (e < k) sa += (vv - mean4[rr]) * (vv - mean4[rr]);
-              }
-              sb += xbe * xbe;
-              if (in) p.xa_out[o * k + e] = vv;
-            }
-#pragma unroll
-            for (int o2 = 1; o2 < 16; o2 <<= 1) {
-              sb += __shfl_xor(sb, o2, 64);
-              sa += __shfl_xor(sa, o2, 64);
-            }
-            if (i16 == 0) {
-              spart[1][wv][vi] = sb;
-              spart[2][wv][vi] = sa;
-            }
-          }
-          __syncthreads();
-          if (wv == 0 && i16 == 0) {
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-              if (sidx4[rr] < 0) continue;
-              const int vi = out_row(rr);
-              const double sb = (spart[1][0][vi] + spart[1][1][vi]) + (spart[1][2][vi] + spart[1][3][vi]);
-              const double sa = (spart[2][0][vi] + spart[2][1][vi]) + (spart[2][2][vi] + spart[2][3][vi]);
-              const long long so = spread_index(p, lo, la, sidx4[rr]);
-              p.spread_b[so] = sqrt(sb / (double)(float)k);
-              p.spread_a[so] = sqrt(sa / (double)(float)k);
-            }
-          }
+          if (st4[rr] < 0) continue;
+          const int vi = out_row(rr);
+          const long long so = spread_index(p, lo, la, st4[rr]);
+          p.spread_b[so] = sqrt(four(sspr[0], vi) / (double)(float)k);
+          p.spread_a[so] = sqrt(four(sspr[EPI ? 1 : 0], vi) / (double)(float)k);
         }
       }
     }

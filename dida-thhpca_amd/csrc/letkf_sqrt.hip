@@ -714,7 +714,7 @@ void k_vec(EigParams p) {
   if (p.xb || p.xb32) {
     // the B operand of the update over the reflector block (consumed by now;
     // the last block's reflectors were staged before the barriers above); for
-    // the FP32 state at k <= 64 in FP32 (the update rounds it to FP32 anyway)
+    // the FP32 state in FP32 (the update rounds it to FP32 anyway)
     float* const rf = reinterpret_cast<float*>(refl);
 #pragma unroll
     for (int I = 0; I < TT; ++I)
@@ -725,7 +725,7 @@ void k_vec(EigParams p) {
         for (int J = 0; J < CPW; ++J) {
           const double v = S[I][J][r] + wf;
           const int o = tile_off<KMAX>(I, w * CPW + J, r, lane);
-          if (KMAX < 128 && p.state_f32) rf[o] = (float)v;
+          if (p.state_f32) rf[o] = (float)v;
           else refl[o] = v;
         }
       }

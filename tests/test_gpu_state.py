@@ -309,3 +309,30 @@ def test_run_da_device_nan_fails():
         with pytest.raises(engine.DidaError, match="background NaN in 1 state elements"):
             eng.run_da_device(xi.data_ptr(), 90.0, 0.0, 1.0, xo.data_ptr(), sb.data_ptr(),
                               sa.data_ptr())
+
+
+@pytest.mark.parametrize("k,nz,halo,f32", [
+    (65, 2, 0, 1), (66, 5, 1, 1), (68, 10, 0, 1), (100, 5, 0, 1), (127, 16, 0, 1),
+    (128, 11, 2, 1), (65, 5, 0, 0), (90, 10, 1, 0), (128, 16, 0, 0)])
+def test_update_of_wide_ensembles(k, nz, halo, f32):
+    """The update of k = 65..128 at ensemble widths with whole and partial
+    16-byte pieces, and at numbers of state vectors around its groups of 16."""
+    import torch
+    import orc
+    from dida_letkf import synth
+    inst = synth.generate("c3", seed=k, k=k, nlat=5, nlon=9, nz=nz, n_obs=4000,
+                          halo=halo, local_dist=900.0)
+    ref = orc.letkf_compute(inst)
+    eng = _engine(inst, 0)
+    dt = np.float32 if f32 else np.float64
+    xb, axb = _dev(inst.xb, dt), _dev(inst.axb)
+    xa, axa = torch.zeros_like(xb), torch.zeros_like(axb)
+    f = eng.analyze_device_f32 if f32 else eng.analyze_device
+    assert f(xb.data_ptr(), axb.data_ptr(), xa.data_ptr(), axa.data_ptr()) == 0
+    torch.cuda.synchronize()
+    xa, axa = xa.cpu().numpy().astype(np.float64), axa.cpu().numpy()
+    if f32:
+        err = increment_error(inst, xa + axa[..., None], ref["xa"] + ref["axa"][..., None])
+        assert max(err.values()) < 1e-5
+    else:
+        assert rel(xa, ref["xa"]) < TOL64 and rel(axa, ref["axa"]) < TOL64
