@@ -2474,26 +2474,40 @@ hipError_t launch_split(hipStream_t st, const SplitParams& p) {
   return hipGetLastError();
 }
 
-// One workgroup per column (halo columns included: they are zeroed, as
-// letkf_compute.F90:191-193 zeroes xa and axa before the loop); wavefront w
-// takes the state elements v = w, w + 4, ...  For each covering cube in loop
-// order (lon cubes outer, lat cubes inner), lane e forms
-// dist(e) = axb(v) + sum_m xb(m, v) trans(m, e) (xb(m, v) broadcast from lane
-// m), the wavefront sums dist for the mean, and the lane adds dist(e) - mean
-// to xa(e, v) and the mean to axa(v) (xb_add2_xa, letkf_compute.F90:332-382);
-// the column is then divided by its cube count (:248-255).
-template <int KM>
-__global__ __launch_bounds__(256) void k_overlap_update(OverlapParams p) {
-  constexpr int R = KM / 64;            // members per lane
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// One wavefront per column and group of 16 state elements (halo columns
+// included: they are zeroed, as letkf_compute.F90:191-193 zeroes xa and axa
+// before the loop).  xb_add2_xa (letkf_compute.F90:332-382) adds, for each
+// covering cube c, the members dist_c(e) - mean_e dist_c and the mean itself,
+// dist_c(e) = axb(v) + sum_m xb(m, v) trans_c(m, e), and the column is divided
+// by its cube count (:248-255).  The sums over m and c are one FP64 MFMA
+// chain per 16 members (16 elements x k by k x 16, over all covering cubes);
+// axb is left out of it and enters the mean only, so the members lose no
+// digits to its size.  A lane's operands of two consecutive steps are two
+// consecutive members of its element (A) and of its trans column (B), one
+// 16-byte load.
+// The bound is the load latency of trans (L2).  (A lane per member, each
+// streaming its trans column against broadcasts of xb, used k of 64 lanes and
+// one chain of k FMAs: 96x48, k = 20, 25 elements, 4 cubes a column, 379 us
+// there; now 34 us.)
+template <int KMAX>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KMAX == 32 ? 4 : KMAX == 64 ? 3 : 2)))
+void k_overlap_update(OverlapParams p, int ngrp,
+                                                        long long n_items) {
+  constexpr int TT = KMAX / 16, S2 = KMAX / 8;   // member tiles, pairs of steps
+  const int lane = threadIdx.x & 63, i16 = lane & 15, q = lane >> 4;
+  const long long item = (long long)blockIdx.x * 4 + uniform((int)(threadIdx.x >> 6));
+  if (item >= n_items) return;
+  const long long col = item / ngrp;
+  const int v0 = 16 * (int)(item % ngrp);
   const int lat_ext = p.g.nlat + 2 * p.halo;
-  const int la_e = blockIdx.x % lat_ext, lo_e = blockIdx.x / lat_ext;
+  const int la_e = (int)(col % lat_ext), lo_e = (int)(col / lat_ext);
   const int k = p.k, n = p.n;
-  const long long off = ((long long)lo_e * lat_ext + la_e) * n;
+  const long long off = col * n;
   const int la = la_e - p.halo, lo = lo_e - p.halo;
   if (la < 0 || la >= p.g.nlat || lo < 0 || lo >= p.g.nlon) {
-    for (int i = threadIdx.x; i < n * k; i += blockDim.x) p.xa[off * k + i] = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) p.axa[off + i] = 0.0;
+    const int nv = min(16, n - v0);
+    for (int i = lane; i < nv * k; i += 64) p.xa[(off + v0) * k + i] = 0.0;
+    if (lane < nv) p.axa[off + v0 + lane] = 0.0;
     return;
   }
   const int cn = p.g.cube_n, cs = p.g.cube_s;
@@ -2504,67 +2518,102 @@ __global__ __launch_bounds__(256) void k_overlap_update(OverlapParams p) {
   const int jc1 = min(lo / cs, p.g.nlon_c - 1);
   const double count = (double)((ic1 - ic0 + 1) * (jc1 - jc0 + 1));
   const long long kk = (long long)k * k;
-  for (int v = wave; v < n; v += 4) {
-    const double* xbc = p.xb + (off + v) * k;
-    const double ab = p.axb[off + v];
-    double xv[R], acc[R];
+  // steps 2 s and 2 s + 1 of lane quarter q carry members 8 s + 2 q and the
+  // next: one load of both (8-byte aligned) from the whole blocks of 8, the
+  // block that k cuts read member by member, one in its place past k - 1
+  // (they meet zeros in A)
+  typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+  const int kf = k / 8, cut0 = min(8 * kf + 2 * q, k - 1), cut1 = min(8 * kf + 2 * q + 1, k - 1);
+  auto pairs = [&](const double* base, double (&x)[S2][2]) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int e = lane + 64 * r;
-      xv[r] = e < k ? xbc[e] : 0.0;
-      acc[r] = 0.0;
-    }
-    double accm = 0.0;
-    for (int jc = jc0; jc <= jc1; ++jc) {
-      for (int ic = ic0; ic <= ic1; ++ic) {
-        const long long c = (long long)jc * p.g.nlat_c + ic;
-        const bool keep = p.status[c] != 0;
-        double dist[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const int e = lane + 64 * r;
-          const double* tr = p.trans + c * kk + (long long)(e < k ? e : 0) * k;
-          double s = 0.0;
-          if (keep) {
-            s = xv[r];
-          } else {
-#pragma unroll
-            for (int rr = 0; rr < R; ++rr)
-              for (int m = 0; m < min(64, k - 64 * rr); ++m)
-                s = fma(__shfl(xv[rr], m, 64), tr[64 * rr + m], s);
-          }
-          dist[r] = e < k ? ab + s : 0.0;
-        }
-        double sum = 0.0;
-#pragma unroll
-        for (int r = 0; r < R; ++r) sum += dist[r];
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
-        const double mean = sum / k;
-        accm += mean;
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] += dist[r] - mean;
+    for (int s = 0; s < S2; ++s) {
+      if (s < kf) {
+        const d2 t = *reinterpret_cast<const d2*>(base + 2 * q + 8 * s);
+        x[s][0] = t.x;
+        x[s][1] = t.y;
+      } else if (8 * s < k) {
+        x[s][0] = base[cut0];
+        x[s][1] = base[cut1];
       }
     }
+  };
+  double xv[S2][2] = {};
+  const int va = v0 + i16;
+  pairs(p.xb + (off + min(va, n - 1)) * k, xv);
+#pragma unroll
+  for (int s = 0; s < S2; ++s)
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+      xv[s][x] = va < n && 8 * s + 2 * q + x < k ? xv[s][x] : 0.0;
+  d4 acc[TT];
+#pragma unroll
+  for (int J = 0; J < TT; ++J) acc[J] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int jc = jc0; jc <= jc1; ++jc) {
+    for (int ic = ic0; ic <= ic1; ++ic) {
+      const long long c = (long long)jc * p.g.nlat_c + ic;
+      if (p.status[c] != 0) {                    // trans = I
+#pragma unroll
+        for (int J = 0; J < TT; ++J) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int v = v0 + q + 4 * r, e = 16 * J + i16;
+            if (v < n && e < k) acc[J][r] += p.xb[(off + v) * k + e];
+          }
+          asm volatile("" ::: "memory");
+        }
+        continue;
+      }
+      const double* tr = p.trans + c * kk;
+#pragma unroll
+      for (int J = 0; J < TT; ++J) {
+        if (16 * J >= k) continue;
+        double b[S2][2] = {};
+        pairs(tr + min(16 * J + i16, k - 1) * k, b);
+#pragma unroll
+        for (int s = 0; s < S2; ++s) {
+          if (8 * s >= k) continue;
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+            acc[J] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[s][x], b[s][x], acc[J], 0, 0, 0);
+        }
+        // the next tile's loads stay behind this one's: all of them at once
+        // take the registers of other wavefronts
+        asm volatile("" ::: "memory");
+      }
+    }
+  }
+  // lane holds element v0 + q + 4 r, member 16 J + i16 (0 past k - 1)
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int v = v0 + q + 4 * r;
+    double sum = 0.0;
+#pragma unroll
+    for (int J = 0; J < TT; ++J) sum += 16 * J + i16 < k ? acc[J][r] : 0.0;
+    sum += dpp_d<0xB1>(sum);
+    sum += dpp_d<0x4E>(sum);
+    sum += dpp_d<0x141>(sum);
+    sum += dpp_d<0x140>(sum);
+    const double mean = sum / k;
+    if (v >= n) continue;
     double* xac = p.xa + (off + v) * k;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int e = lane + 64 * r;
-      if (e < k) xac[e] = acc[r] / count;
+    for (int J = 0; J < TT; ++J) {
+      const int e = 16 * J + i16;
+      if (e < k) xac[e] = (acc[J][r] - mean) / count;
     }
-    if (lane == 0) p.axa[off + v] = accm / count;
+    if (i16 == 0) p.axa[off + v] = p.axb[off + v] + mean / count;
   }
 }
 
 hipError_t launch_overlap_update(hipStream_t st, const OverlapParams& p) {
   const long long cols = (long long)(p.g.nlat + 2 * p.halo) * (p.g.nlon + 2 * p.halo);
-  if (cols <= 0) return hipSuccess;
-  if (p.k <= 64)
-    hipLaunchKernelGGL(k_overlap_update<64>, dim3((unsigned)cols), dim3(256), 0, st, p);
-  else if (p.k <= 128)
-    hipLaunchKernelGGL(k_overlap_update<128>, dim3((unsigned)cols), dim3(256), 0, st, p);
-  else
-    return hipErrorInvalidValue;
+  const int ngrp = (p.n + 15) / 16;
+  const long long items = cols * ngrp;
+  const dim3 grid((unsigned)((items + 3) / 4));
+  if (p.k <= 32) hipLaunchKernelGGL(k_overlap_update<32>, grid, dim3(256), 0, st, p, ngrp, items);
+  else if (p.k <= 64) hipLaunchKernelGGL(k_overlap_update<64>, grid, dim3(256), 0, st, p, ngrp, items);
+  else if (p.k <= 128) hipLaunchKernelGGL(k_overlap_update<128>, grid, dim3(256), 0, st, p, ngrp, items);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

@@ -180,3 +180,23 @@ def test_overlap_argument_checks():
         xa, axa = torch.zeros_like(xb), torch.zeros_like(axb)
         with pytest.raises(engine.DidaError, match="FP64 state"):
             eng.analyze_device_f32(xb.data_ptr(), axb.data_ptr(), xa.data_ptr(), axa.data_ptr())
+
+
+@pytest.mark.parametrize("k,nz,cn,ov,halo", [
+    (2, 1, 3, 2, 0), (7, 5, 4, 3, 1), (9, 2, 2, 1, 0), (31, 5, 3, 1, 0), (33, 10, 5, 2, 2),
+    (63, 2, 4, 2, 0), (70, 5, 3, 2, 0), (127, 2, 3, 1, 1)])
+def test_overlap_update_widths(k, nz, cn, ov, halo):
+    """Ensemble widths around the update's blocks of 8 and 16 members, state
+    vectors around its groups of 16."""
+    import orc
+    from dida_letkf import synth
+    if nz == 1:
+        inst = synth.generate("c0", seed=90 + k, k=k, nlat=9, nlon=14, n_obs=900, halo=halo,
+                              local_dist=900.0)
+    else:
+        inst = synth.generate("c2", seed=90 + k, k=k, nlat=9, nlon=14, nz=nz, n_obs=3000,
+                              halo=halo, local_dist=900.0)
+    inst.cfg.cube_n, inst.cfg.overlap = cn, ov
+    ref = orc.letkf_compute(inst, want_trans=True)
+    got = _run(inst, precision=0, keep=True)
+    assert rel(got["xa"], ref["xa"]) < TOL64 and rel(got["axa"], ref["axa"]) < TOL64
