@@ -1994,7 +1994,13 @@ int core_run(hipStream_t st, CoreBufs& cb, EigScratch& es, int mode, int k, long
   pp.h0 = 0;
   pp.A = cb.A.as<double>();
   pp.b = cb.b.as<double>();
-  HIP_TRY(launch_products(st, pp, precision));
+  // One wavefront per analysis leaves most of the 1,024 SIMDs idle below that
+  // many analyses, and each list is a chain; in parts, from two steps of rows
+  // a wavefront on (k = 64, 1,000 rows: 199 -> 47 us; 256 of k = 40: 92 -> 26)
+  if (precision == DIDA_PREC_FP64 && n_an <= 1024 && nr >= 32 * n_an)
+    HIP_TRY(launch_products_parts(st, pp));
+  else
+    HIP_TRY(launch_products(st, pp, precision));
   XformParams xp{};
   xp.g = g;
   xp.k = k;

@@ -368,6 +368,9 @@ hipError_t launch_list_counts(hipStream_t st, const long long* off, int n_list, 
                               long long* total);
 hipError_t launch_zero_ll(hipStream_t st, long long* p, long long n);
 hipError_t launch_select_tile(hipStream_t st, const SelectParams& p, bool fill);
+// FP64 products of n_an single columns (nzc = 1, no order list), each list in
+// parts over the wavefronts of a workgroup
+hipError_t launch_products_parts(hipStream_t st, const ProdParams& p);
 hipError_t launch_products(hipStream_t st, const ProdParams& p, int precision);
 // bucket schedule over the positions [p.seg_lo, p.seg_hi) of p.order: in
 // dispatch order, or on a persistent work queue when p.q_counter is set

@@ -569,20 +569,20 @@ struct PairTable {
   __device__ static constexpr int J(int pid) { return pid - I(pid) * (I(pid) + 1) / 2; }
 };
 
+// tiles [WS PPW, ...) of an analysis and, for WS = 0, b: the sums over rows
+// [r0, r1) (products_f64_rows) and their store (products_f64_store)
 template <int KP, int WS, int PPW, bool PW>
-__device__ __forceinline__ void products_f64_wave(const ProdParams& p, long long a, int ah,
-                                                  double vc, long long r0, long long r1,
-                                                  int lane) {
+__device__ __forceinline__ void products_f64_rows(const ProdParams& p, double vc, long long r0,
+                                                  long long r1, int lane, d4 (&acc)[PPW],
+                                                  double (&bacc)[KP / 16]) {
   constexpr int T = KP / 16;
   using PT = PairTable<T>;
   constexpr int P0 = WS * PPW;
   constexpr int P1 = (P0 + PPW < PT::N) ? P0 + PPW : PT::N;
   constexpr int NP = P1 - P0;
   const int i16 = lane & 15, q = lane >> 4;
-  d4 acc[NP];
 #pragma unroll
-  for (int x = 0; x < NP; ++x) acc[x] = d4{0.0, 0.0, 0.0, 0.0};
-  double bacc[T];
+  for (int x = 0; x < PPW; ++x) acc[x] = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int t = 0; t < T; ++t) bacc[t] = 0.0;
   // G groups of 4 rows per step (lane q takes rows 4g + q), loaded one step
@@ -644,6 +644,18 @@ __device__ __forceinline__ void products_f64_wave(const ProdParams& p, long long
       }
     }
   }
+}
+
+template <int KP, int WS, int PPW>
+__device__ __forceinline__ void products_f64_store(const ProdParams& p, long long a, int lane,
+                                                   const d4 (&acc)[PPW],
+                                                   const double (&bacc)[KP / 16]) {
+  constexpr int T = KP / 16;
+  using PT = PairTable<T>;
+  constexpr int P0 = WS * PPW;
+  constexpr int P1 = (P0 + PPW < PT::N) ? P0 + PPW : PT::N;
+  constexpr int NP = P1 - P0;
+  const int i16 = lane & 15, q = lane >> 4;
   double* A = p.A + (a - p.a0) * (long long)KP * KP;
 #pragma unroll
   for (int x = 0; x < NP; ++x) {
@@ -665,6 +677,16 @@ __device__ __forceinline__ void products_f64_wave(const ProdParams& p, long long
       if (q == 0) b[16 * t + i16] = v;
     }
   }
+}
+
+template <int KP, int WS, int PPW, bool PW>
+__device__ __forceinline__ void products_f64_wave(const ProdParams& p, long long a, int ah,
+                                                  double vc, long long r0, long long r1,
+                                                  int lane) {
+  d4 acc[PPW];
+  double bacc[KP / 16];
+  products_f64_rows<KP, WS, PPW, PW>(p, vc, r0, r1, lane, acc, bacc);
+  products_f64_store<KP, WS, PPW>(p, a, lane, acc, bacc);
 }
 
 template <int KP, int SCHED, bool PW>
@@ -690,6 +712,69 @@ __global__ __launch_bounds__(256) void k_products_f64(ProdParams p) {
       if (wsub == 3) products_f64_wave<KP, 3, PPW, PW>(p, a, ah, vc, r0, r1, lane);
     }
   });
+}
+
+// A few analyses on their own (letkf_core): a workgroup of eight wavefronts
+// takes one, NR of them contiguous parts of its row list each (KP = 128: two
+// parts of four wavefronts), and the parts' sums meet in LDS pair by pair,
+// part h + i into part i.  A single list is a chain of row gathers: one
+// wavefront took 199 us for 1,000 rows of k = 64, and 92 us for 256 analyses
+// of up to 400 rows of k = 40; now 47 and 26 us (bound: the f64 MFMAs of one
+// CU, 17 us of them for the 1,000 rows).
+template <int KP>
+__global__ __launch_bounds__(512) void k_products_parts(ProdParams p) {
+  constexpr int T = KP / 16;
+  constexpr int NPAIR = T * (T + 1) / 2;
+  constexpr int WPA = (NPAIR + 9) / 10;
+  constexpr int PPW = (NPAIR + WPA - 1) / WPA;
+  constexpr int NR = 8 / WPA;
+  static_assert(WPA == 1 || (WPA == 4 && NPAIR == 4 * PPW), "a wavefront or four per part");
+  __shared__ double red[NR / 2][WPA][PPW * 4 + T][64];
+  const int lane = threadIdx.x & 63, wave = uniform((int)(threadIdx.x >> 6));
+  const int ws = wave % WPA, part = wave / WPA;
+  const long long a = p.a0 + blockIdx.x;
+  const int ah = (int)a;
+  const long long r0 = min(p.row_off[ah - p.h0], p.row_cap);
+  const long long r1 = min(p.row_off[ah - p.h0 + 1], p.row_cap);
+  // parts of whole steps of 8 rows
+  const long long chunk = (r1 - r0 + 8 * NR - 1) / (8 * NR) * 8;
+  const long long s0 = min(r0 + part * chunk, r1), s1 = min(s0 + chunk, r1);
+  d4 acc[PPW];
+  double bacc[T];
+  if (ws == 0) products_f64_rows<KP, 0, PPW, false>(p, 0.0, s0, s1, lane, acc, bacc);
+  if constexpr (WPA > 1) {
+    if (ws == 1) products_f64_rows<KP, 1, PPW, false>(p, 0.0, s0, s1, lane, acc, bacc);
+    if (ws == 2) products_f64_rows<KP, 2, PPW, false>(p, 0.0, s0, s1, lane, acc, bacc);
+    if (ws == 3) products_f64_rows<KP, 3, PPW, false>(p, 0.0, s0, s1, lane, acc, bacc);
+  }
+#pragma unroll
+  for (int h = NR / 2; h >= 1; h /= 2) {
+    if (part >= h && part < 2 * h) {
+#pragma unroll
+      for (int x = 0; x < PPW; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[part - h][ws][4 * x + r][lane] = acc[x][r];
+#pragma unroll
+      for (int t = 0; t < T; ++t) red[part - h][ws][4 * PPW + t][lane] = bacc[t];
+    }
+    __syncthreads();
+    if (part < h) {
+#pragma unroll
+      for (int x = 0; x < PPW; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[x][r] += red[part][ws][4 * x + r][lane];
+#pragma unroll
+      for (int t = 0; t < T; ++t) bacc[t] += red[part][ws][4 * PPW + t][lane];
+    }
+    __syncthreads();
+  }
+  if (part > 0) return;
+  if (ws == 0) products_f64_store<KP, 0, PPW>(p, a, lane, acc, bacc);
+  if constexpr (WPA > 1) {
+    if (ws == 1) products_f64_store<KP, 1, PPW>(p, a, lane, acc, bacc);
+    if (ws == 2) products_f64_store<KP, 2, PPW>(p, a, lane, acc, bacc);
+    if (ws == 3) products_f64_store<KP, 3, PPW>(p, a, lane, acc, bacc);
+  }
 }
 
 template <int KP, int WS, int PPW, bool PW>
@@ -2416,6 +2501,15 @@ hipError_t launch_products(hipStream_t st, const ProdParams& p, int precision) {
   if (p.kp == 64) return launch_products_kp<64>(st, p, precision, nullptr);
   if (p.kp == 128) return launch_products_kp<128>(st, p, precision, nullptr);
   return hipErrorInvalidValue;
+}
+
+hipError_t launch_products_parts(hipStream_t st, const ProdParams& p) {
+  const dim3 grid((unsigned)p.n_an);
+  if (p.kp == 32) hipLaunchKernelGGL(k_products_parts<32>, grid, dim3(512), 0, st, p);
+  else if (p.kp == 64) hipLaunchKernelGGL(k_products_parts<64>, grid, dim3(512), 0, st, p);
+  else if (p.kp == 128) hipLaunchKernelGGL(k_products_parts<128>, grid, dim3(512), 0, st, p);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
 }
 
 hipError_t launch_transform(hipStream_t st, const XformParams& p) {

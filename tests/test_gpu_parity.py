@@ -418,3 +418,27 @@ def test_products_paths_match(pk, prec):
         ref = orc.letkf_compute(inst)
         err = increment_error(inst, gpu["xa"], gpu["axa"], ref["xa"], ref["axa"])
         assert max(err.values()) < 1e-4, err
+
+
+@pytest.mark.parametrize("k", [2, 20, 32, 33, 64, 65, 128])
+def test_letkf_core_lists_in_parts(k):
+    """Row lists split over the wavefronts of a workgroup: from lists shorter
+    than the parts to many steps each, with every remainder of the steps, one
+    list on its own and several ragged ones."""
+    import orc
+    from dida_letkf import engine
+    rng = np.random.default_rng(k)
+    cases = []
+    for p in (0, 1, 7, 8, 9, 31, 63, 64, 65, 130, 515, 1025):
+        Y = rng.standard_normal((k, p))
+        Y -= Y.mean(axis=0, keepdims=True)
+        cases.append((Y, (1.0 / rng.uniform(0.3, 3.0, p) ** 2).astype(np.float32),
+                      rng.standard_normal(p), rng.uniform(0.0, 1.0, p)))
+    t, w, st = engine.letkf_core_batched(*[[c[i] for c in cases] for i in range(4)],
+                                         inflation_factor=1.1)
+    assert np.all(st == 0)
+    for i, c in enumerate(cases):
+        tr, wr = orc.letkf_core(*c, inflation_factor=1.1)[:2]
+        assert rel(t[i], tr) < TOL64 and np.abs(w[i] - wr).max() < 1e-10 * max(1.0, np.abs(wr).max())
+        t1, w1 = engine.letkf_core(*c, inflation_factor=1.1)
+        assert rel(t1, tr) < TOL64 and np.abs(w1 - wr).max() < 1e-10 * max(1.0, np.abs(wr).max())
