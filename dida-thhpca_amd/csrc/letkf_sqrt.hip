@@ -170,8 +170,11 @@ struct SqrtLds {
   static constexpr int N = F > B ? (F > FD ? F : FD) : (B > FD ? B : FD);
 };
 
+// k <= 32: three wavefronts per SIMD hide more of each one's chain than the
+// spills they cost (228 B a lane): 2,073,600 matrices 28 -> 24 ms, four
+// wavefronts 31 ms.  k > 32 spills at two already.
 template <int KMAX, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(KMAX == 32 ? 3 : 2)))
 void k_vec(EigParams p) {
   using Lds = SqrtLds<KMAX, NW>;
   constexpr int TT = Lds::TT, NP = Lds::NP, LDP = Lds::LDP, LDV = Lds::LDV, LDT = Lds::LDT;
