@@ -42,101 +42,156 @@ __device__ __forceinline__ double grid_weight(const float* __restrict__ g, int n
   return (d - v + (double)ga) / d;
 }
 
-__device__ __forceinline__ double ph_mid(const ObsOpParams& p, int l, double ps) {
+// Pressure of the faces and mid-levels of the hybrid coordinate
+// (vert_coord_mod.F90:556-561) from {hyai (p0 - ptop), hybi} per face.
+__device__ __forceinline__ double ph_face(const ObsOpParams& p, double2 c, double ps) {
 #pragma clang fp contract(off)
-  // mid-level l (1-based) of the hybrid coordinate (vert_coord_mod.F90:556-561);
-  // level nz + 1 repeats level nz
-  if (l > p.nz) l = p.nz;
-  const double a = p.hyai[l - 1] * (p.p0 - p.ptop) + p.hybi[l - 1] * (ps - p.ptop) + p.ptop;
-  const double b = p.hyai[l] * (p.p0 - p.ptop) + p.hybi[l] * (ps - p.ptop) + p.ptop;
-  return 0.5 * (a + b);
+  return c.x + c.y * (ps - p.ptop) + p.ptop;
 }
 
-template <int MEMB>
+// Faces whose coefficients a workgroup keeps in LDS; more are read in memory.
+constexpr int kFacesLds = 256;
+
+// SITES sites per wavefront (1, or 4 where that still fills the chip): the
+// grid cells of all of them are found at once, lane 2 i searching the
+// latitudes and lane 2 i + 1 the longitudes of the i-th, so the chain of
+// dependent reads of a search is paid once for them; then they run one after
+// another, lane = member (neighbours of the list in one wavefront left
+// profiles that stand together to a few wavefronts: 497 and 1,115 us).  The hybrid coefficients come from LDS, each face
+// read once (the next level's upper face is this one's lower).
+// The bound is the gathers: 8 x 8 k bytes a 3-D row from rows nobody shares
+// (360x180x32, k = 64, 296k rows: 1.6 GB).  One site per wavefront with its
+// own searches, every face read from memory twice, took 790 us there, 1,004
+// on its own; now 448 and 624.
+template <int MEMB, int SITES>
 __global__ __launch_bounds__(256) void k_obs_operator(ObsOpParams p) {
 #pragma clang fp contract(off)
-  const int lane = threadIdx.x & 63;
-  const int s = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (s >= p.n_sites) return;
-  const int k = p.k, n = p.n, h = p.halo;
-  int tx = grid_index(p.glat, p.nlat, 90.0f, p.site_lat[s]);
-  int ty = grid_index(p.glon, p.nlon, 360.0f, p.site_lon[s]);
-  const double ax = grid_weight(p.glat, p.nlat, 90.0f, tx, p.site_lat[s]);
-  const double ay = grid_weight(p.glon, p.nlon, 360.0f, ty, p.site_lon[s]);
-  const long long lat_ext = p.nlat + 2 * h;
-  // state offsets of the points (tx-1 | tx) x (ty-1 | ty)
-  const long long o00 = ((long long)(ty - 2 + h) * lat_ext + (tx - 2 + h)) * n;
-  const long long o10 = ((long long)(ty - 2 + h) * lat_ext + (tx - 1 + h)) * n;
-  const long long o01 = ((long long)(ty - 1 + h) * lat_ext + (tx - 2 + h)) * n;
-  const long long o11 = ((long long)(ty - 1 + h) * lat_ext + (tx - 1 + h)) * n;
-  auto bil = [&](int el, int e) -> double {
-    const double x00 = p.xb[(o00 + el) * k + e] + p.axb[o00 + el];
-    const double x10 = p.xb[(o10 + el) * k + e] + p.axb[o10 + el];
-    const double x01 = p.xb[(o01 + el) * k + e] + p.axb[o01 + el];
-    const double x11 = p.xb[(o11 + el) * k + e] + p.axb[o11 + el];
-    const double r1 = x00 * ax + x10 * (1 - ax);
-    const double r2 = x01 * ax + x11 * (1 - ax);
-    return r1 * ay + r2 * (1 - ay);
+  __shared__ double2 sface[kFacesLds];
+  const bool in_lds = p.nz + 1 <= kFacesLds;
+  auto face_of = [&](int l) {
+    return double2{p.hyai[l] * (p.p0 - p.ptop), p.hybi[l]};
   };
-  double ps[MEMB];
-  int jp[MEMB];
-#pragma unroll
-  for (int m = 0; m < MEMB; ++m) {
-    const int e = lane + 64 * m;
-    ps[m] = (e < k) ? bil(p.ps_index, e) : 1.0e5;
-    jp[m] = 1;
+  if (in_lds)
+    for (int l = threadIdx.x; l <= p.nz; l += blockDim.x) sface[l] = face_of(l);
+  __syncthreads();
+  // face l (0-based) for the lane's ps
+  auto face = [&](int l, double ps) { return ph_face(p, in_lds ? sface[l] : face_of(l), ps); };
+  // mid-level l (1-based); level nz + 1 repeats level nz
+  auto ph_mid = [&](int l, double ps) {
+    l = min(l, p.nz);
+    return 0.5 * (face(l - 1, ps) + face(l, ps));
+  };
+  const int lane = threadIdx.x & 63;
+  const int wave = uniform((int)(threadIdx.x >> 6));
+  // the i-th site of wavefront w is w + i n_waves, from the end of the list
+  // that has the longer site (a profile is one chain of rows: begun last it
+  // would run on its own)
+  const int n_waves = (p.n_sites + SITES - 1) / SITES;
+  const int w = blockIdx.x * 4 + wave;
+  if (w >= n_waves) return;
+  const bool from_end = SITES > 1 && p.site_row_ptr[p.n_sites] - p.site_row_ptr[p.n_sites - 1] >
+                                         p.site_row_ptr[1] - p.site_row_ptr[0];
+  auto site = [&](int i) { return w + (from_end ? SITES - 1 - i : i) * n_waves; };
+  const int k = p.k, n = p.n, h = p.halo;
+  int t_l = 1;
+  double w_l = 0.0;
+  {
+    const int s = min(site((lane >> 1) % SITES), p.n_sites - 1);
+    const bool lon = lane & 1;
+    const float* __restrict__ g = lon ? p.glon : p.glat;
+    const int gn = lon ? p.nlon : p.nlat;
+    const float close = lon ? 360.0f : 90.0f;
+    const double v = lon ? p.site_lon[s] : p.site_lat[s];
+    t_l = grid_index(g, gn, close, v);
+    w_l = grid_weight(g, gn, close, t_l, v);
   }
-  // rows outside [0, n_rows) are skipped; a row with an unknown variable
-  // gets NaN (bad input never reads outside the state arrays)
-  const int r0 = max(p.site_row_ptr[s], 0), r1 = min(p.site_row_ptr[s + 1], p.n_rows);
-  for (int r = r0; r < r1; ++r) {
-    const int v = p.row_var[r];
-    if (v < 0 || v >= p.n_var) {
+  const long long lat_ext = p.nlat + 2 * h;
+#pragma unroll 1
+  for (int i = 0; i < SITES; ++i) {
+    const int s = site(i);
+    if (s >= p.n_sites) continue;
+    const int tx = __builtin_amdgcn_readlane(t_l, 2 * i), ty = __builtin_amdgcn_readlane(t_l, 2 * i + 1);
+    const double ax = readlane_d(w_l, 2 * i), ay = readlane_d(w_l, 2 * i + 1);
+    // state offsets of the points (tx-1 | tx) x (ty-1 | ty)
+    const long long o00 = ((long long)(ty - 2 + h) * lat_ext + (tx - 2 + h)) * n;
+    const long long o10 = ((long long)(ty - 2 + h) * lat_ext + (tx - 1 + h)) * n;
+    const long long o01 = ((long long)(ty - 1 + h) * lat_ext + (tx - 2 + h)) * n;
+    const long long o11 = ((long long)(ty - 1 + h) * lat_ext + (tx - 1 + h)) * n;
+    auto bil = [&](int el, int e) -> double {
+      const double x00 = p.xb[(o00 + el) * k + e] + p.axb[o00 + el];
+      const double x10 = p.xb[(o10 + el) * k + e] + p.axb[o10 + el];
+      const double x01 = p.xb[(o01 + el) * k + e] + p.axb[o01 + el];
+      const double x11 = p.xb[(o11 + el) * k + e] + p.axb[o11 + el];
+      const double r1 = x00 * ax + x10 * (1 - ax);
+      const double r2 = x01 * ax + x11 * (1 - ax);
+      return r1 * ay + r2 * (1 - ay);
+    };
+    double ps[MEMB];
+    int jp[MEMB];
+#pragma unroll
+    for (int m = 0; m < MEMB; ++m) {
+      const int e = lane + 64 * m;
+      ps[m] = (e < k) ? bil(p.ps_index, e) : 1.0e5;
+      jp[m] = 1;
+    }
+    // rows outside [0, n_rows) are skipped; a row with an unknown variable
+    // gets NaN (bad input never reads outside the state arrays)
+    const int r0 = max(p.site_row_ptr[s], 0), r1 = min(p.site_row_ptr[s + 1], p.n_rows);
+    for (int r = r0; r < r1; ++r) {
+      const int v = p.row_var[r];
+      if (v < 0 || v >= p.n_var) {
+#pragma unroll
+        for (int m = 0; m < MEMB; ++m) {
+          const int e = lane + 64 * m;
+          if (e < k) p.yb[(long long)r * k + e] = __builtin_nan("");
+        }
+        if (lane == 0) p.dep[r] = __builtin_nan("");
+        continue;
+      }
+      const int vs = p.var_start[v] - 1;
+      const bool three_d = p.var_lev[v] > 1;
+      const double pr = p.row_ph[r];
+      double val[MEMB];
+      double sum = 0.0;
 #pragma unroll
       for (int m = 0; m < MEMB; ++m) {
         const int e = lane + 64 * m;
-        if (e < k) p.yb[(long long)r * k + e] = __builtin_nan("");
-      }
-      if (lane == 0) p.dep[r] = __builtin_nan("");
-      continue;
-    }
-    const int vs = p.var_start[v] - 1;
-    const bool three_d = p.var_lev[v] > 1;
-    const double pr = p.row_ph[r];
-    double val[MEMB];
-    double sum = 0.0;
-#pragma unroll
-    for (int m = 0; m < MEMB; ++m) {
-      const int e = lane + 64 * m;
-      double x = 0.0;
-      if (e < k) {
-        int j = jp[m];
-        while (j <= p.nz && pr > ph_mid(p, j, ps[m])) ++j;
-        jp[m] = j;
-        const int pos = j - 1;
-        if (three_d) {
-          if (pos >= 1 && pos < p.nz) {
-            const int tl = vs + pos - 1;
-            const double lu = log(ph_mid(p, pos + 1, ps[m])), ll = log(ph_mid(p, pos, ps[m]));
-            const double t3 = (lu - log(pr)) / (lu - ll);
-            x = bil(tl, e) * t3 + bil(tl + 1, e) * (1 - t3);
-          } else {
-            x = bil(pos == 0 ? vs : vs + p.nz - 1, e);
+        double x = 0.0;
+        if (e < k) {
+          int j = jp[m];
+          double up = face(j - 1, ps[m]);
+          while (j <= p.nz) {
+            const double lw = face(j, ps[m]);
+            if (!(pr > 0.5 * (up + lw))) break;
+            up = lw;
+            ++j;
           }
-        } else {
-          x = bil(vs, e);
+          jp[m] = j;
+          const int pos = j - 1;
+          if (three_d) {
+            if (pos >= 1 && pos < p.nz) {
+              const int tl = vs + pos - 1;
+              const double lu = log(ph_mid(pos + 1, ps[m])), ll = log(ph_mid(pos, ps[m]));
+              const double t3 = (lu - log(pr)) / (lu - ll);
+              x = bil(tl, e) * t3 + bil(tl + 1, e) * (1 - t3);
+            } else {
+              x = bil(pos == 0 ? vs : vs + p.nz - 1, e);
+            }
+          } else {
+            x = bil(vs, e);
+          }
         }
+        val[m] = x;
+        sum += x;
       }
-      val[m] = x;
-      sum += x;
-    }
-    const double mean = wave_sum(sum) / k;
+      const double mean = wave_sum(sum) / k;
 #pragma unroll
-    for (int m = 0; m < MEMB; ++m) {
-      const int e = lane + 64 * m;
-      if (e < k) p.yb[(long long)r * k + e] = val[m] - mean;
+      for (int m = 0; m < MEMB; ++m) {
+        const int e = lane + 64 * m;
+        if (e < k) p.yb[(long long)r * k + e] = val[m] - mean;
+      }
+      if (lane == 0) p.dep[r] = p.yo[r] - mean;
     }
-    if (lane == 0) p.dep[r] = p.yo[r] - mean;
   }
 }
 
@@ -187,13 +242,21 @@ hipError_t launch_fill_halo(hipStream_t st, double* x, int nlat, int nlon, int h
   return hipGetLastError();
 }
 
-hipError_t launch_obs_operator(hipStream_t st, const ObsOpParams& p) {
-  if (p.n_sites <= 0) return hipSuccess;
-  const unsigned blocks = (unsigned)((p.n_sites + 3) / 4);
-  if (p.k <= 64) hipLaunchKernelGGL(k_obs_operator<1>, dim3(blocks), dim3(256), 0, st, p);
-  else if (p.k <= 128) hipLaunchKernelGGL(k_obs_operator<2>, dim3(blocks), dim3(256), 0, st, p);
+template <int SITES>
+static hipError_t launch_obs_operator_s(hipStream_t st, const ObsOpParams& p) {
+  const unsigned blocks = (unsigned)((p.n_sites + 4LL * SITES - 1) / (4LL * SITES));
+  if (p.k <= 64) hipLaunchKernelGGL((k_obs_operator<1, SITES>), dim3(blocks), dim3(256), 0, st, p);
+  else if (p.k <= 128) hipLaunchKernelGGL((k_obs_operator<2, SITES>), dim3(blocks), dim3(256), 0, st, p);
   else return hipErrorInvalidValue;
   return hipGetLastError();
+}
+
+hipError_t launch_obs_operator(hipStream_t st, const ObsOpParams& p) {
+  if (p.n_sites <= 0) return hipSuccess;
+  // four sites a wavefront from the count on whose wavefronts still fill the
+  // chip (256 CUs of 32): 201k sites 789 -> 375..448 us; below it a site's own
+  // chain is what a call waits for (40 of them: 23 -> 20 us a call)
+  return p.n_sites >= 4 * 8192 ? launch_obs_operator_s<4>(st, p) : launch_obs_operator_s<1>(st, p);
 }
 
 }  // namespace dida

@@ -176,3 +176,31 @@ def test_obs_records_through_operator_and_analysis():
     r = (ref["xa"] + ref["axa"][..., None])[h:-h, h:-h]
     print("records -> operator -> analysis", _rel(g, r))
     assert _rel(g, r) < TOL
+
+
+@pytest.mark.parametrize("k,nz,n_obs,first", [(8, 6, 32768, 0), (20, 5, 32801, 1), (70, 4, 33003, 0),
+                                              (5, 300, 400, 0), (5, 254, 33000, 1)])
+def test_obs_operator_many_sites(k, nz, n_obs, first):
+    """Several sites per wavefront, profiles last or first in the list, every
+    remainder of the sites, and more levels than the coefficient table holds."""
+    import dataclasses
+    import orc
+    from dida_letkf import synth, engine
+    c = synth.obs_operator_case("c2", seed=200 + k, k=k, nlat=10, nlon=21, nz=nz, n_obs=n_obs,
+                                n_stations=7, n_ps=60)
+    if first:                         # the sites in reverse order
+        rp = c.site_row_ptr
+        idx = np.concatenate([np.arange(rp[s], rp[s + 1]) for s in range(len(rp) - 2, -1, -1)])
+        c = dataclasses.replace(
+            c, site_lat=c.site_lat[::-1].copy(), site_lon=c.site_lon[::-1].copy(),
+            site_row_ptr=np.concatenate([[0], np.cumsum(np.diff(rp)[::-1])]).astype(rp.dtype),
+            row_var=c.row_var[idx], row_ph=c.row_ph[idx], yo=c.yo[idx])
+    yb_o, dep_o = orc.obs_operator(c)
+    yb_g, dep_g = engine.obs_operator(c)
+    H_o = yb_o + (c.yo - dep_o)[:, None]
+    H_g = yb_g + (c.yo - dep_g)[:, None]
+    print(k, nz, c.site_lat.size, _rel(H_g, H_o), flush=True)
+    assert _rel(H_g, H_o) < TOL
+    for rows in (c.row_var == 0, c.row_var != 0):
+        assert np.abs(yb_g[rows] - yb_o[rows]).max() <= TOL * np.abs(H_o[rows]).max()
+        assert np.abs(dep_g[rows] - dep_o[rows]).max() <= TOL * np.abs(H_o[rows]).max()
