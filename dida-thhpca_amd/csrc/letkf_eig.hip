@@ -1535,20 +1535,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   if (p.w_out && h == 0 && in_r) p.w_out[a * (long long)k + r] = sw[r];
 }
 
+// Exchanges the upper 32 lanes of x with the lower 32 of y, and the odd rows of
+// 16 lanes of x with the even rows of y: together, over four registers, the
+// transposition between registers and lane quarters.
+__device__ __forceinline__ void swap_halves(float& x, float& y) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  x = __uint_as_float(r[0]);
+  y = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_rows(float& x, float& y) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  x = __uint_as_float(r[0]);
+  y = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_halves(double&, double&) {}
+__device__ __forceinline__ void swap_rows(double&, double&) {}
+
 // Xa = Xb trans for k = 65..128: wave w produces members 32w .. 32w+31, its
 // trans columns (128 x 32) in registers; all four take the same groups of 16
 // state vectors.  TS and EPI as k_update.
 //
 // The bound is the state and trans in HBM (10.7 GB for the FP32 state of
 // 64,800 columns of 97 vectors at k = 128) and the f32 MFMAs beside it.  A
-// operands come straight from the state: the MFMA reduction index is permuted
-// so that a lane's operands are 16-byte pieces of its vector (step s, lane
-// quarter q carry member 4 VEC (s / VEC) + VEC q + s mod VEC, so one load
-// instruction covers 64 contiguous bytes of each of 16 vectors), the next
-// group's as soon as the MFMAs have consumed this one's; LDS only carries the
-// wavefronts' shares of the means, one barrier a group.  (Staged through LDS
+// operands come straight from the state in 16-byte pieces, one load instruction
+// covering 64 contiguous bytes of each of 16 vectors, the next group's as soon
+// as the MFMAs have consumed this one's.  FP64 permutes the reduction index to
+// the pieces (step s, lane quarter q carry member 8 (s / 2) + 2 q + s mod 2);
+// FP32, whose sums would round differently, transposes four pieces between the
+// lane quarters instead (v_permlane swaps) and keeps members 4 s + q.  LDS only
+// carries the wavefronts' shares of the means, one barrier a group.  (Staged through LDS
 // between two barriers a group, with no load in flight across them, and sums
-// by shuffles, 10.7 ms there; now 4.3 ms.)
+// by shuffles, 10.7 ms there; now about 6.4, cycle 63.1 ms; FP32 in the order of
+// the pieces 4.3 and 61.0 ms.)
 template <class TS, int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_update128(EigParams p) {
@@ -1574,20 +1592,21 @@ void k_update128(EigParams p) {
   // q + 4 rr for f64 16x16x4, 4 q + rr for f32 16x16x4
   constexpr bool F32 = sizeof(TS) == 4;
   auto out_row = [q](int rr) { return F32 ? 4 * q + rr : q + 4 * rr; };
-  auto member = [q](int s) { return 4 * VEC * (s / VEC) + VEC * q + s % VEC; };
+  auto piece = [q](int s) { return 4 * VEC * (s / VEC) + VEC * q + s % VEC; };
+  auto member = [q, piece](int s) { return F32 ? 4 * s + q : piece(s); };
   const TS* __restrict__ xb = ST::xb(p);
   // trans tiles from the transform, in the state's precision
   const TS* __restrict__ tb =
       reinterpret_cast<const TS*>(p.refl + ai * (long long)kp * kp);
   // tile_off of member(s)'s row, split in the lane's part and a constant
   const TS* __restrict__ tl =
-      tb + tile_off<KMAX>(0, 2 * wv, F32 ? q : q >> 1, (F32 ? 0 : 32 * (q & 1)) + i16);
+      tb + tile_off<KMAX>(0, 2 * wv, F32 ? 0 : q >> 1, F32 ? lane : 32 * (q & 1) + i16);
   TS bop[S][2];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
 #pragma unroll
     for (int J = 0; J < 2; ++J)
-      bop[s][J] = tl[tile_off<KMAX>(s >> 2, J, F32 ? 0 : s & 2, 16 * (F32 ? s & 3 : s & 1))];
+      bop[s][J] = tl[tile_off<KMAX>(s >> 2, J, F32 ? s & 3 : s & 2, F32 ? 0 : 16 * (s & 1))];
     if (s % 8 == 7) __builtin_amdgcn_sched_barrier(0);
   }
 
@@ -1636,11 +1655,18 @@ void k_update128(EigParams p) {
 #pragma unroll
       for (int s = 0; s < SA; s += VEC) {
         // an in-row load and a select: no branch
-        const int m = member(s0 + s);
+        const int m = piece(s0 + s);
         const uint4 t4 = *reinterpret_cast<const uint4*>(xr + (m < k ? m : 0));
         const TS* tv = reinterpret_cast<const TS*>(&t4);
 #pragma unroll
         for (int x = 0; x < VEC; ++x) af[s + x] = (s_a >= 0 && m < k) ? tv[x] : (TS)0;
+        // register x of quarter q: member 16 (s / 4) + 4 q + x -> 4 x + q
+        if constexpr (F32) {
+          swap_halves(af[s], af[s + 2]);
+          swap_halves(af[s + 1], af[s + 3]);
+          swap_rows(af[s], af[s + 1]);
+          swap_rows(af[s + 2], af[s + 3]);
+        }
       }
     } else {
 #pragma unroll

@@ -940,9 +940,13 @@ __global__ __launch_bounds__(256) void k_products_f32(ProdParams p) {
 // weight at one of the wavefront's levels in a ring, in list order, and the
 // weights, the gathers and the MFMAs take blocks of 64 kept rows.  A row with
 // weight 0 adds exact zeros unless its Yb, d or R^-1 is not finite: obs sets
-// that hold such a value (obs_bad) keep every row.
+// that hold such a value (obs_bad) keep every row.  FP64 keeps rows one by one.
+// FP32, whose sums would round differently in another grouping, keeps whole
+// groups of 4 list positions (an MFMA step, a row per lane quarter), and every
+// row of the lists that flush: the same bits as with no row left out.
 // 360x180x32, k = 32, 3.2 G rows, FP32: 138 ms with weights beside the MFMAs,
-// 55 ms with blocks of 64 unfiltered rows, 22 ms now (cycle 108 -> 77 ms).
+// 55 ms with blocks of 64 unfiltered rows, about 40 ms now (cycle 91 ms; row by
+// row 22 and 72).
 template <class REAL> struct LevelReal;
 template <> struct LevelReal<double> {
   using acc = d4;
@@ -1008,7 +1012,7 @@ __device__ __forceinline__ void products_levels_wave(const ProdParams& p, long l
   // 2 vert_dist, so a row it drops has |vc - vco| / vert_dist > 2 however the
   // division rounds; a NaN coordinate is kept
   const double lim = 2.0 * p.vert_dist * (1.0 + 1e-12);
-  const bool keep_all = *p.obs_bad != 0;
+  const bool keep_all = *p.obs_bad != 0 || (sizeof(REAL) == 4 && n > kFlushMinRows);
   const unsigned long long below = (1ull << lane) - 1;
   int scan = 0, head = 0, pend = 0, fr0 = 0, fr1 = 0;
   double fv0 = 0.0;
@@ -1023,7 +1027,15 @@ __device__ __forceinline__ void products_levels_wave(const ProdParams& p, long l
 #pragma unroll
       for (int v = 0; v < LV; ++v) keep = keep || !(fabs(vc[v] - fv0) > lim);
       keep = keep && scan + lane < n;
-      const unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
+      unsigned long long m = __builtin_amdgcn_ballot_w64(keep);
+      if constexpr (sizeof(REAL) == 4) {
+        // whole groups of 4
+        m |= m >> 1;
+        m |= m >> 2;
+        m = (m & 0x1111111111111111ull) * 15;
+        keep = (m >> lane & 1) && scan + lane < n;
+        m = __builtin_amdgcn_ballot_w64(keep);
+      }
       if (keep) {
         const int s = (head + pend + __popcll(m & below)) & 127;
         sh.pend_row[s] = fr0;

@@ -1,6 +1,6 @@
 // letkf_obsop.hip -- observation operator H and Yb/d centring on device.
 //
-// One wavefront per obs site, lane e = member e (members e and e + 64 for
+// A wavefront takes a site at a time, lane e = member e (members e and e + 64 for
 // k > 64).  Per site: the grid cell (find_obs_grid, letkf_obs.F90:192-248),
 // each member's pressure profile from its interpolated ps
 // (ps2ph_3d_interp, obs_make.F90:345-381), then per row the bilinear value,
