@@ -1,5 +1,6 @@
 // letkf_eig.hip -- the transform of a batch of local analyses and the ensemble
-// update: tridiagonalisation, the QL list pass, the update, and the launches.
+// update: tridiagonalisation, the QL of indefinite matrices, the update, and the
+// launches.
 //
 // The k x k matrices M = A + (k-1)/rho I of one batch are reduced to
 // tridiagonal form, and trans and overline_w follow from that form:
@@ -15,11 +16,18 @@
 // k = 65..128 runs k_tridiag128 and k_update128 with half rows per thread
 // (256 threads per matrix).
 //
-// A matrix whose M is not positive definite, or not finite, is flagged
-// (status != 0) and appended to a device-side list; k_update skips it.  The
-// list pass then diagonalises it by implicit QL with Wilkinson shift (Golub &
-// Van Loan Alg. 8.3.1, Sec. 8.3.5; Bowdler, Martin, Reinsch & Wilkinson
-// 1968) from the stored tridiagonal form, with no host synchronisation:
+// A matrix whose M is finite but not positive definite goes to k_indef, which
+// diagonalises it by implicit QL with Wilkinson shift (Golub & Van Loan Alg.
+// 8.3.1, Sec. 8.3.5; Bowdler, Martin, Reinsch & Wilkinson 1968) from its
+// tridiagonal form, before the update and with no host synchronisation.  An
+// analysis whose QL does not converge, or whose M or overline_w is not finite,
+// leaves xa = xb, axa = axb for its state and NaN in trans/overline_w; the
+// caller gets the count.
+//
+// With the QL limits lowered from the environment (EigParams::ql_first) the
+// first pass is the QL recurrence for every matrix, so that its flag paths can
+// be tested; the matrices it flags go to a device-side list and a second,
+// list pass with twice the limits:
 //
 //   k_ql_log    one LANE per matrix (64 matrices per wavefront): the scalar
 //               QL recurrence, which is a serial chain per matrix; writes the
@@ -30,11 +38,8 @@
 //               then overline_w = V diag(1/lambda) V^T b and
 //               trans = V diag(sqrt((k-1)/lambda)) V^T + overline_w 1^T
 //               (letkf_core.F90:129-225) on f64 MFMA
-// An analysis still flagged after it (QL not converged, or its rotation log
-// full) leaves xa = xb, axa = axb for its state and NaN in trans/overline_w;
-// the caller gets the count.  With the QL limits lowered from the environment
-// (EigParams::ql_first) the first pass is the QL recurrence for every matrix,
-// so that its flag paths can be tested.
+#include <algorithm>
+
 #include "letkf_device.h"
 #include "letkf_kernels.h"
 #include "letkf_eig.h"
@@ -393,7 +398,7 @@ __device__ __forceinline__ double block2_min(double v, double* red, int& slot) {
 }
 
 // ---------------------------------------------------------------------------
-// k_rot (list pass): V (Q accumulation, logged rotations), overline_w and
+// k_rot (ql_first): V (Q accumulation, logged rotations), overline_w and
 // trans = T + overline_w 1^T with LDS staged in small chunks, trans written
 // in the register layout of the update's MFMA B operand over the analysis'
 // reflector block (consumed by then), as k_vec does.  k_update streams the
@@ -446,8 +451,7 @@ void k_rot(EigParams p) {
   static_assert(REFILL >= KMAX + 16 && REFILL % 64 == 0, "a refill covers any chase");
   __shared__ __align__(16) double sbuf[L::N];
   // stage C's vectors share one array with stage A's Gram matrices (16 x 16),
-  // which are dead by then: k_rot<64> then needs 11.4 KB of LDS, so eight of
-  // its workgroups and one of k_ql_log's (66.5 KB) fit a CU together
+  // which are dead by then
   constexpr int NSC = 5 * KMAX > 256 ? 5 * KMAX : 256;
   __shared__ double ssc[NSC], stau[KMAX];
   double* const sf = ssc;
@@ -746,6 +750,164 @@ void k_rot(EigParams p) {
   if (p.w_out && in_r) p.w_out[a * (long long)k + lane] = wbar;
 }
 
+// ---------------------------------------------------------------------------
+// k_indef: the matrices k_vec found finite but not positive definite
+// (kStatusIndefinite: R^-1 < 0, or an M so ill conditioned that its smallest
+// eigenvalue is rounding), by QL with Wilkinson shift from their tridiagonal
+// form, as k_ql_log and k_rot, however many there are.
+// ---------------------------------------------------------------------------
+// A workgroup takes every gridDim-th matrix of the batch that carries the
+// status: thread 0 runs the QL recurrence a chase at a time, thread r applies
+// the chase's rotations to row r of Z in LDS.  Rare, so plain (a log of the
+// rotations, which k_ql_log keeps per matrix, would be four times the matrix);
+// a batch without such a matrix pays the launch and one read.
+// Runs before the update, which then takes every analysis in one pass.
+template <int KMAX>
+__global__ __launch_bounds__(KMAX < 64 ? 64 : KMAX) void k_indef(EigParams p) {
+  if (*p.flag_n == 0) return;
+  __shared__ double sZ[KMAX * KMAX];                 // column-major: Z(r, c) at c KMAX + r
+  __shared__ double sd[KMAX], se[KMAX], sv[KMAX], sb[KMAX], sw[KMAX];
+  __shared__ double2 srot[KMAX];                     // (c, s) of position i of the chase
+  __shared__ int s_lo, s_hi, s_end;                  // the chase; s_end: no chase left
+  const int r = threadIdx.x;
+  const bool row = r < KMAX;
+  const int k = p.k, kp = p.kp;
+  const double eps = 2.220446049250313e-16;
+  for (long long al = blockIdx.x; al < p.n_an; al += gridDim.x) {
+    const long long a = p.a0 + al;
+    if (p.status[a] != kStatusIndefinite) continue;
+    double* refl = p.refl + al * (long long)kp * kp;
+    if (row) {
+      sd[r] = r < k ? p.d[al * kp + r] : 0.0;
+      se[r] = r + 1 < k ? p.e[al * kp + r] : 0.0;
+      sb[r] = r < k ? p.b[al * kp + r] : 0.0;
+      for (int c = 0; c < KMAX; ++c) sZ[c * KMAX + r] = c == r ? 1.0 : 0.0;
+    }
+    // Z = Q = H_0 .. H_(k-3)
+    for (int j = 0; j + 2 < k; ++j) {
+      __syncthreads();
+      if (row) sv[r] = refl[(long long)j * kp + r];
+      __syncthreads();
+      if (row) {
+        double dot = 0.0;
+        for (int c = j + 1; c < k; ++c) dot = fma(sZ[c * KMAX + r], sv[c], dot);
+        dot *= p.tau[al * kp + j];
+        for (int c = j + 1; c < k; ++c) sZ[c * KMAX + r] = fma(-dot, sv[c], sZ[c * KMAX + r]);
+      }
+    }
+    __syncthreads();
+    double tnorm = 0.0;
+    for (int i = 0; i < k; ++i) tnorm = fmax(tnorm, fabs(sd[i]) + fabs(se[i]));
+    int l = 0, iter = 0, status = 0;                 // thread 0's
+    for (;;) {
+      if (r == 0) {
+        s_lo = s_hi = 0;
+        s_end = 0;
+        // the first l that is not an eigenvalue yet, and its block l .. m
+        int m = l;
+        for (; l < k; ++l, iter = 0) {
+          for (m = l; m < k - 1; ++m) {
+            const double em = fabs(se[m]);
+            if (em <= eps * (fabs(sd[m]) + fabs(sd[m + 1])) || em <= eps * tnorm) break;
+          }
+          if (m > l) break;
+        }
+        if (l < k && ++iter > p.max_iter) status = l + 1;
+        if (l >= k || status != 0) {
+          s_end = 1;
+        } else {
+          double g = (sd[l + 1] - sd[l]) / (2.0 * se[l]);
+          double t = hypot(g, 1.0);
+          g = sd[m] - sd[l] + se[l] / (g + (g >= 0.0 ? fabs(t) : -fabs(t)));
+          double s = 1.0, c = 1.0, pp = 0.0;
+          int i = m - 1;
+          for (; i >= l; --i) {
+            const double f = s * se[i], bb = c * se[i];
+            const double r2 = fma(f, f, g * g);
+            const double rinv = rsqrt(r2);
+            if (r2 == 0.0) {                         // underflow: the chase stops here
+              se[i + 1] = 0.0;
+              sd[i + 1] -= pp;
+              break;
+            }
+            se[i + 1] = r2 * rinv;
+            s = f * rinv;
+            c = g * rinv;
+            g = sd[i + 1] - pp;
+            t = (sd[i] - g) * s + 2.0 * c * bb;
+            pp = s * t;
+            sd[i + 1] = g + pp;
+            g = c * t - bb;
+            srot[i] = make_double2(c, s);
+          }
+          s_lo = i + 1;
+          s_hi = m;
+          if (i < l) {
+            sd[l] -= pp;
+            se[l] = g;
+          }
+          se[m] = 0.0;
+        }
+      }
+      __syncthreads();
+      if (s_end) break;
+      if (row) {
+        const int lo = s_lo, hi = s_hi;
+        double carry = sZ[hi * KMAX + r];
+        for (int i = hi - 1; i >= lo; --i) {
+          const double2 cs = srot[i];
+          const double z = sZ[i * KMAX + r];
+          sZ[(i + 1) * KMAX + r] = fma(cs.x, carry, cs.y * z);
+          carry = fma(-cs.y, carry, cs.x * z);
+        }
+        sZ[lo * KMAX + r] = carry;
+      }
+      __syncthreads();
+    }
+    // functions of the eigenvalues (letkf_core.F90:107-113, the guard of the
+    // reduced precisions): sv = sqrt((k-1)/lambda), sw = 1/lambda V^T b
+    double lmin = 0.0;
+    if (p.guard)
+      for (int i = 0; i < k; ++i) lmin = fmin(lmin, sd[i]);
+    if (row) {
+      const double lam = r < k ? sd[r] - lmin + (double)(k - 1) / p.inflation : 1.0;
+      double tb = 0.0;
+      for (int i = 0; i < k; ++i) tb = fma(sZ[r * KMAX + i], sb[i], tb);
+      sv[r] = r < k ? sqrt((double)(k - 1) / lam) : 0.0;
+      sw[r] = r < k ? tb / lam : 0.0;
+    }
+    __syncthreads();
+    double w = 0.0;
+    if (r < k)
+      for (int c = 0; c < k; ++c) w = fma(sZ[c * KMAX + r], sw[c], w);
+    const bool bad = __syncthreads_or((r == 0 && status != 0) || !__builtin_isfinite(w));
+    if (r == 0) p.status[a] = status != 0 ? status : bad ? kStatusNonFinite : 0;
+    if (bad) {
+      nan_transform(p, a);
+    } else {
+      if (p.w_out && r < k) p.w_out[a * (long long)k + r] = w;
+      // trans(f, e) = T(f, e) + overline_w(f) (letkf_core.F90:221-225), f = r;
+      // for the update in the layout k_vec leaves, zero past k
+      float* const rf = reinterpret_cast<float*>(refl);
+      if (row)
+        for (int e = 0; e < KMAX; ++e) {
+          double t = 0.0;
+          if (r < k && e < k) {
+            for (int c = 0; c < k; ++c) t = fma(sZ[c * KMAX + r] * sv[c], sZ[c * KMAX + e], t);
+            t += w;
+            if (p.trans_out) p.trans_out[a * (long long)k * k + (long long)e * k + r] = t;
+          }
+          if (p.xb || p.xb32) {
+            const int o = tile_off<KMAX>(r >> 4, e >> 4, (r & 15) >> 2, 16 * (r & 3) + (e & 15));
+            if (p.state_f32) rf[o] = (float)t;
+            else refl[o] = t;
+          }
+        }
+    }
+    __syncthreads();
+  }
+}
+
 // State precision of the update: FP64 (xb/xa) or FP32 (xb32/xa32) members on
 // f64 or f32 MFMA 16x16x4 (the two share their operand layout).
 template <class TS> struct StateT;
@@ -773,9 +935,14 @@ __device__ __forceinline__ long long spread_index(const EigParams& p, int lo, in
   return ((long long)(lo - 1) * p.g.nlat + (la - 1)) * p.n + v;
 }
 
-// An analysis whose eigensolve failed on both passes (or found no room in the
-// list pass): its state rows keep the background -- xa = xb, axa = axb, or
-// with the fused epilogue xa_out = xb + axb and spread_a = spread_b.
+// True when the update is the last word on an analysis with a nonzero status,
+// so that its state rows keep the background; false when the list pass follows.
+__device__ __forceinline__ bool keeps_background(const EigParams& p, int status) {
+  return p.list || !p.ql_first || status == kStatusNotRedone || status == kStatusNonFinite;
+}
+
+// A failed analysis: xa = xb, axa = axb, or with the fused epilogue
+// xa_out = xb + axb and spread_a = spread_b.
 template <class TS, int EPI>
 __device__ void copy_background_t(const EigParams& p, long long a) {
   const AnRows R = an_rows(p, a);
@@ -862,8 +1029,8 @@ void k_update(EigParams p) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   long long a, ai, ar;
   if (!eig_slot(p, blockIdx.x, a, ai, ar)) return;
-  if (p.status[a] != 0) {                // redone by the list pass, or failed
-    if (p.list || keeps_background(p.status[a])) copy_background_t<TS, EPI>(p, a);
+  if (p.status[a] != 0) {                // failed, or redone by the list pass
+    if (keeps_background(p, p.status[a])) copy_background_t<TS, EPI>(p, a);
     return;
   }
   const int k = p.k;
@@ -1582,8 +1749,8 @@ void k_update128(EigParams p) {
   const int lane = tid & 63, wv = tid >> 6;
   long long a, ai, ar;
   if (!eig_slot(p, blockIdx.x, a, ai, ar)) return;
-  if (p.status[a] != 0) {                // redone by the list pass, or failed
-    if (p.list || keeps_background(p.status[a])) copy_background_t<TS, EPI>(p, a);
+  if (p.status[a] != 0) {                // failed, or redone by the list pass
+    if (keeps_background(p, p.status[a])) copy_background_t<TS, EPI>(p, a);
     return;
   }
   const int k = p.k, kp = p.kp;
@@ -1903,8 +2070,7 @@ static void launch_update(hipStream_t st, const EigParams& p, unsigned nb) {
 
 // one of the four stages over the batch p: tridiagonalisation; the guard's
 // smallest eigenvalue (reduced precision); trans and overline_w; update.  With
-// ql_first stages 1 and 2 are the list pass's kernels, the QL recurrence and
-// its rotations.
+// ql_first stages 1 and 2 are the QL recurrence and its rotations.
 template <int KMAX>
 static void launch_eig_stage_k(hipStream_t st, const EigParams& p, int stage) {
   const unsigned nb = (unsigned)p.n_an;
@@ -1917,6 +2083,9 @@ static void launch_eig_stage_k(hipStream_t st, const EigParams& p, int stage) {
     if (has_state(p)) launch_update<KMAX>(st, p, nb);
   } else if (!p.ql_first) {
     (void)launch_sqrt(st, p, stage == 1);
+    if (stage == 2)
+      hipLaunchKernelGGL(k_indef<KMAX>, dim3((unsigned)std::min(p.n_an, 256LL)),
+                         dim3(KMAX < 64 ? 64 : KMAX), 0, st, p);
   } else if (stage == 1) {
     hipLaunchKernelGGL(k_ql_log<KMAX>, dim3(nq), dim3(64), 0, st, p);
   } else {

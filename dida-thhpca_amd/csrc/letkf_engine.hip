@@ -300,19 +300,14 @@ size_t eig_bytes_per_analysis(int k) {
   return sizeof(double) * ((size_t)kp * kp + 4 * kp);
 }
 
-// QL iterations per eigenvalue before a matrix is flagged (first pass; the
-// list pass allows twice as many), as the EISPACK/Numerical Recipes QL does
+// QL iterations per eigenvalue before a matrix is flagged (first QL pass; the
+// list pass and k_indef allow twice as many), as the EISPACK/Numerical Recipes
+// QL does
 constexpr int kQlMaxIter = 30;
 
-// Analyses the list pass can redo per batch, and its per-analysis scratch
-// (a rotation log and chase log twice the first pass's)
+// Analyses the list pass can redo per batch
 long long rerun_cap_of(int k, long long n_an) {
   return std::min<long long>(n_an, k > 64 ? 128 : 256);
-}
-size_t rerun_bytes_per_slot(int k) {
-  const int kp = kp_of(k);
-  return 16 * (size_t)(2 * rot_cap_of(k)) + 16 * (size_t)(2 * kHdrCapPerK * k) + sizeof(int) +
-         sizeof(double) * kp + sizeof(int);
 }
 
 // Optional positive integer from the environment (0 when unset).  The QL
@@ -325,11 +320,15 @@ int env_int(const char* name) {
   return std::max(0, std::atoi(e));
 }
 
-// The first pass takes the QL recurrence only where its limits are set.
+// The first pass takes the QL recurrence, and a list pass follows, only where
+// its limits are set.
 bool ql_first() { return env_int("DIDA_ROT_CAP") || env_int("DIDA_QL_MAXITER"); }
 
-// Sizes every eigensolver buffer for batches of up to n analyses (the list
-// pass's too), so that the launches of a call allocate nothing.
+// ints of the flag counts and, with ql_first, the list of the list pass
+long long flag_ints(int k, long long n_an) { return 2 + (ql_first() ? rerun_cap_of(k, n_an) : 0); }
+
+// Sizes every eigensolver buffer for batches of up to n analyses, so that the
+// launches of a call allocate nothing.
 int eig_prepare(EigScratch& s, int k, long long n) {
   const int kp = kp_of(k);
   const long long cap = rerun_cap_of(k, n);
@@ -342,24 +341,24 @@ int eig_prepare(EigScratch& s, int k, long long n) {
     RC_TRY(s.rot.ensure((size_t)16 * n * rot_cap_of(k)));
     RC_TRY(s.hdr.ensure((size_t)16 * n * kHdrCapPerK * k));
     RC_TRY(s.nchase.ensure(sizeof(int) * n));
+    RC_TRY(s.rr_rot.ensure((size_t)16 * cap * 2 * rot_cap_of(k)));
+    RC_TRY(s.rr_hdr.ensure((size_t)16 * cap * 2 * kHdrCapPerK * k));
+    RC_TRY(s.rr_nchase.ensure(sizeof(int) * cap));
+    RC_TRY(s.rr_lam.ensure(sizeof(double) * cap * kp));
   }
-  RC_TRY(s.flags.ensure(sizeof(int) * (2 + cap)));
-  RC_TRY(s.rr_rot.ensure((size_t)16 * cap * 2 * rot_cap_of(k)));
-  RC_TRY(s.rr_hdr.ensure((size_t)16 * cap * 2 * kHdrCapPerK * k));
-  RC_TRY(s.rr_nchase.ensure(sizeof(int) * cap));
-  RC_TRY(s.rr_lam.ensure(sizeof(double) * cap * kp));
+  RC_TRY(s.flags.ensure(sizeof(int) * flag_ints(k, n)));
   return DIDA_OK;
 }
 
 // Zeroes the call-wide flag count; run once per analysis call.
 int eig_begin_call(hipStream_t st, EigScratch& s, int k, long long max_batch) {
-  RC_TRY(s.flags.ensure(sizeof(int) * (2 + rerun_cap_of(k, max_batch))));
+  RC_TRY(s.flags.ensure(sizeof(int) * flag_ints(k, max_batch)));
   HIP_TRY(launch_zero_ints(st, s.flags.as<int>(), 2));
   return DIDA_OK;
 }
 
-// Eigensolver parameters of the batch xp (its scratch allocated): the split
-// eigensolver (k_tridiag, k_ql_log, k_vec + k_update) over analyses
+// Transform parameters of the batch xp (its scratch allocated): the split
+// transform (k_tridiag, k_lmin, k_vec, k_indef, k_update) over analyses
 // [xp.a0, xp.a0 + xp.n_an).
 int prepare_eig(EigScratch& s, const XformParams& xp, EigParams& ep) {
   const long long n = xp.n_an;
@@ -378,8 +377,7 @@ int prepare_eig(EigScratch& s, const XformParams& xp, EigParams& ep) {
     RC_TRY(s.hdr.ensure((size_t)16 * n * hdr_cap));
     RC_TRY(s.nchase.ensure(sizeof(int) * n));
   }
-  const long long rcap = rerun_cap_of(k, n);
-  if (s.flags.bytes < sizeof(int) * (2 + rcap))
+  if (s.flags.bytes < sizeof(int) * flag_ints(k, n))
     return set_error(DIDA_ERR_STATE, "eigensolver flags not set up for this batch");
   ep = EigParams{};
   ep.g = xp.g;
@@ -388,11 +386,12 @@ int prepare_eig(EigScratch& s, const XformParams& xp, EigParams& ep) {
   ep.inflation = xp.inflation;
   ep.guard = xp.guard;
   ep.ql_first = ql;
-  ep.max_iter = env_int("DIDA_QL_MAXITER") ? env_int("DIDA_QL_MAXITER") : kQlMaxIter;
+  ep.max_iter = 2 * kQlMaxIter;
+  if (ql) ep.max_iter = env_int("DIDA_QL_MAXITER") ? env_int("DIDA_QL_MAXITER") : kQlMaxIter;
   ep.flag_n = s.flags.as<int>();
   ep.flag_total = s.flags.as<int>() + 1;
-  ep.flag_list = s.flags.as<int>() + 2;
-  ep.flag_cap = (int)rcap;
+  ep.flag_list = ql ? s.flags.as<int>() + 2 : nullptr;
+  ep.flag_cap = ql ? (int)rerun_cap_of(k, n) : 0;
   ep.list = nullptr;
   ep.list_n = nullptr;
   ep.list_cap = 0;
@@ -445,8 +444,8 @@ int prepare_eig(EigScratch& s, const XformParams& xp, EigParams& ep) {
   return DIDA_OK;
 }
 
-// The list pass over the analyses the first pass flagged: k_ql_log with a
-// rotation log and an iteration limit twice the first pass's, then k_vec and
+// The list pass over the analyses the first QL pass flagged: k_ql_log with a
+// rotation log and an iteration limit twice the first pass's, then k_rot and
 // k_update, all on st after the first pass (no host synchronisation).
 int rerun_flagged(hipStream_t st, EigScratch& s, const EigParams& ep) {
   const int k = ep.k, kp = ep.kp;
@@ -474,9 +473,9 @@ int rerun_flagged(hipStream_t st, EigScratch& s, const EigParams& ep) {
   return DIDA_OK;
 }
 
-// Transform + update of analyses [xp.a0, xp.a0 + xp.n_an): the split
-// eigensolver, then its list pass over the analyses it flagged; mode 1 runs
-// only the single kernel (k <= 64).
+// Transform + update of analyses [xp.a0, xp.a0 + xp.n_an): the split transform
+// (with ql_first its list pass after it); mode 1 runs only the single kernel
+// (k <= 64).
 // kev: null, or 5 events for the split kernels (recorded only if *split is set)
 int run_transform(hipStream_t st, EigScratch& s, const XformParams& xp, int mode,
                   hipEvent_t* kev = nullptr, bool* split = nullptr) {
@@ -491,7 +490,7 @@ int run_transform(hipStream_t st, EigScratch& s, const XformParams& xp, int mode
   HIP_TRY(launch_zero_ints(st, ep.flag_n, 1));
   HIP_TRY(launch_eig(st, ep, kev));
   if (split) *split = true;
-  return rerun_flagged(st, s, ep);
+  return ep.ql_first ? rerun_flagged(st, s, ep) : DIDA_OK;
 }
 
 // cubes along n grid points with starts every cube_n - overlap (cube_n
@@ -1909,12 +1908,12 @@ int core_layout(CoreBufs& cb, EigScratch& es, int k, long long n_an, long long n
     add(es.rot, 16 * n * (size_t)rot_cap_of(k));
     add(es.hdr, 16 * n * (size_t)(kHdrCapPerK * k));
     add(es.nchase, 4 * n);
+    add(es.rr_rot, 16 * cap * (size_t)(2 * rot_cap_of(k)));
+    add(es.rr_hdr, 16 * cap * (size_t)(2 * kHdrCapPerK * k));
+    add(es.rr_nchase, 4 * cap);
+    add(es.rr_lam, 8 * cap * kp);
   }
-  add(es.flags, 4 * (2 + cap));
-  add(es.rr_rot, 16 * cap * (size_t)(2 * rot_cap_of(k)));
-  add(es.rr_hdr, 16 * cap * (size_t)(2 * kHdrCapPerK * k));
-  add(es.rr_nchase, 4 * cap);
-  add(es.rr_lam, 8 * cap * kp);
+  add(es.flags, 4 * (size_t)flag_ints(k, n_an));
   return c;
 }
 constexpr int kCoreMaxBufs = 32;
@@ -2040,7 +2039,8 @@ void release_core(CoreBufs& cb, EigScratch& es) {
   size_t sizes[kCoreMaxBufs];
   const int nb = core_layout(cb, es, 2, 1, 1, DIDA_PREC_BF16X3, bufs, sizes);
   for (int i = 0; i < nb; ++i) bufs[i]->release();
-  for (DevBuf* b : {&es.rot, &es.hdr, &es.nchase}) b->release();
+  for (DevBuf* b : {&es.rot, &es.hdr, &es.nchase, &es.rr_rot, &es.rr_hdr, &es.rr_nchase, &es.rr_lam})
+    b->release();
 }
 
 // The drop-in letkf_core_ is called once per local analysis (64,800 times a
@@ -2236,7 +2236,6 @@ size_t dida_letkf_job_bytes(const dida_letkf_config* c, int n_sites, int n_rows)
   b += 20 * mb * (size_t)rows_per_column_bound(*c, n_rows);
   b += 16 * (mb + 1) * 2;
   b += mb * nzc * (8 * kp * kp + 8 * kp + eig_bytes_per_analysis(c->k));
-  b += rerun_cap_of(c->k, (long long)(mb * nzc)) * rerun_bytes_per_slot(c->k);
   b += 4 * n_an;
   if (c->keep_transforms) b += n_an * (8 * k * k + 8 * k);
   else b += ovl_trans;                                              // overlapped cubes' trans

@@ -20,17 +20,15 @@ inline int rot_cap_of(int k) { return kRotCapPerK2 * k * k + 16 * k + 64; }
 constexpr int kHdrCapPerK = 8;    // chase log: 8 k chases per analysis
 // eigensolver status per analysis: 0 converged; l + 1 > 0: the QL of
 // eigenvalue l did not converge; kStatusLogFull: the rotation or chase log
-// filled up; kStatusNotRedone: flagged by the first pass when the list pass
-// was full (the analysis keeps its background); kStatusNonFinite: overline_w
-// is not finite (a NaN or Inf in d or R^-1 with a finite A; the analysis
-// keeps its background)
+// filled up; kStatusNotRedone: flagged by the first QL pass when the list pass
+// was full (the analysis keeps its background); kStatusNonFinite: A or
+// overline_w is not finite (a NaN or Inf in Yb, d or R^-1; the analysis keeps
+// its background); kStatusIndefinite: between k_vec and k_indef, M is finite
+// but k_vec found it not positive definite
 constexpr int kStatusLogFull = -1;
 constexpr int kStatusNotRedone = -2;
 constexpr int kStatusNonFinite = -3;
-// the update keeps the background of an analysis with this first-pass status
-__host__ __device__ inline bool keeps_background(int status) {
-  return status == kStatusNotRedone || status == kStatusNonFinite;
-}
+constexpr int kStatusIndefinite = -4;
 
 struct Geom {
   const float* glat;   // nlat, real(4) degrees
@@ -229,13 +227,15 @@ struct EigParams {
   int guard;
   int max_iter;             // QL iterations per eigenvalue before the matrix is flagged
   long long a0, n_an;
-  // Flag list.  First pass (list == NULL): k_vec (or k_ql_log, ql_first)
-  // appends every analysis it flags to flag_list (global index, at most flag_cap entries; *flag_n
-  // counts all of them, *flag_total accumulates over the batches of a call).
-  // Rerun pass (list != NULL): the kernels take analysis list[slot] for
-  // slot < min(*list_n, list_cap); batch-local inputs (d, e, refl, tau, b) are
-  // indexed by list[slot] - a0, the pass's own scratch (rot, hdr, nchase, lam)
-  // by slot.
+  // *flag_n counts the analyses of the batch that k_vec leaves to k_indef, and
+  // *flag_total, over the batches of a call, all that k_vec found not positive
+  // definite or not finite.
+  // Flag list (ql_first).  First pass (list == NULL): k_ql_log appends every
+  // analysis it flags to flag_list (global index, at most flag_cap entries) and
+  // counts it in both.  Rerun pass (list != NULL): the kernels take analysis
+  // list[slot] for slot < min(*list_n, list_cap); batch-local inputs (d, e,
+  // refl, tau, b) are indexed by list[slot] - a0, the pass's own scratch (rot,
+  // hdr, nchase, lam) by slot.
   int* flag_list;
   int* flag_n;
   int* flag_total;
@@ -256,7 +256,7 @@ struct EigParams {
   int4* hdr;                // batch-local, hdr_cap chases (lo, hi, off) per analysis
   int rot_cap, hdr_cap;
   int ql_first;             // the first pass is the QL recurrence (rot, hdr, nchase sized for
-                            // the batch) instead of k_vec
+                            // the batch) and a list pass follows, instead of k_vec and k_indef
   int tridiag_lds;          // k <= 64: tridiagonalise in LDS (1) or in VGPRs (0)
   int* nchase;              // batch-local
   int* status;              // global index
@@ -392,7 +392,8 @@ hipError_t launch_fill_halo(hipStream_t st, double* x, int nlat, int nlon, int h
 // zeroes the halo columns of such a field
 hipError_t launch_zero_halo(hipStream_t st, double* x, int nlat, int nlon, int halo, long long inner);
 hipError_t launch_eig(hipStream_t st, const EigParams& p, hipEvent_t* ev = nullptr);
-// second pass over the analyses the first flagged (p.list / p.list_n / p.list_cap)
+// ql_first: second pass over the analyses the first flagged (p.list / p.list_n /
+// p.list_cap)
 hipError_t launch_eig_rerun(hipStream_t st, const EigParams& p);
 // the guard's smallest eigenvalue (guard_pass; nothing without p.guard), or
 // trans and overline_w, of the batch p from its tridiagonal form

@@ -27,8 +27,8 @@
 //      products Y and X move through no LDS.
 //   4. overline_w = T (T b) / (k-1).
 //
-// It replaces the QL recurrence and the product of its rotations (k_ql_log and
-// k_rot, now the list pass), ~4,500 dependent Givens steps per matrix at k = 64
+// It replaces the QL recurrence and the product of its rotations (k_indef keeps
+// them for M not positive definite), ~4,500 dependent Givens steps per matrix at k = 64
 // and 6 k flops for each.  64,800 matrices: k = 64, 3.95 + 7.25 -> 0.21
 // (k_lmin) + 2.40 ms; k = 128, 50 + 80 -> 0.5 + 20 ms; and a single matrix of
 // k = 64 takes 60 us here against 1.3 ms.  Bound: the wavefront's own chain
@@ -226,7 +226,7 @@ void k_vec(EigParams p) {
   // negative rounding is small; it is checked beside the first poles' pivots
   // (lane NP tests that D - m has positive pivots), and where it fails the
   // largest (0.9 / 2^t) (k-1)/rho that holds is taken.  None holding: D is not
-  // positive definite, or not finite, and the list pass takes the matrix.
+  // positive definite, and k_indef takes the matrix, or it is not finite.
   double m = 0.9 * m0, L = 0.0, qn = 0.0;
   int N = 0;
   // pivots of the poles c0 .. c0 + NP - 1, one lane per pole (wavefront 0); a
@@ -324,13 +324,17 @@ void k_vec(EigParams p) {
     const unsigned long long bal = __builtin_amdgcn_ballot_w64(pos);
     const int f = bal ? __builtin_ctzll(bal) : 64;
     if (f > 50 || !(bound < 1e290) || m < 0.9 * m0) {
+      // k_indef takes a finite matrix; nothing comes of one that is not
+      bool fin = true;
+      for (int i = lane; i < k; i += 64)
+        fin = fin && __builtin_isfinite(p.d[al * kp + i]) && __builtin_isfinite(p.e[al * kp + i]);
+      fin = __builtin_amdgcn_ballot_w64(!fin) == 0;
       if (tid == 0) {
-        p.status[a] = 1;
-        const int s = atomicAdd(p.flag_n, 1);
-        if (s < p.flag_cap) p.flag_list[s] = (int)a;
-        else p.status[a] = kStatusNotRedone;
+        p.status[a] = fin ? kStatusIndefinite : kStatusNonFinite;
+        if (fin) atomicAdd(p.flag_n, 1);
         atomicAdd(p.flag_total, 1);
       }
+      if (!fin) nan_transform(p, a);
       return;
     }
     m = 0.9 * m0 * exp2(-1.0 - (double)f);

@@ -17,7 +17,8 @@
  * handle's stream.
  *
  * Errors: functions return DIDA_OK (0), a negative DIDA_ERR_* code, or, from
- * the analysis calls, a positive count of analyses whose eigensolve failed
+ * the analysis calls, a positive count of analyses whose eigensolve failed or
+ * whose obs terms are not finite
  * (the reference prints dsyevd's ierr and continues, letkf_core.F90:119-122);
  * those analyses leave the background in place and give NaN transforms.
  * dida_letkf_last_error() gives the message of the last failure on the
@@ -123,8 +124,9 @@ typedef struct dida_letkf_stats {
                                reduced precisions */
     double ms_apply;        /* of ms_transform: inverse square root and transform kernel */
     double ms_update;       /* of ms_transform: ensemble update kernel (0 when fused) */
-    int n_rerun;            /* analyses the transform's first pass flagged (M not positive
-                               definite or not finite) and its list pass redid by QL */
+    int n_rerun;            /* analyses whose M is not positive definite (they are
+                               diagonalised by QL) or not finite (they keep their
+                               background) */
     /* Products schedule.  Length buckets over the local obs count p of a
      * column: [0] p = 0, [1] 1..256, [2] 257..512, ... [6] 4097..8192, [7] more. */
     int schedule;                    /* 1: buckets + persistent work queue; 0: column order */

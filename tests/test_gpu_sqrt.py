@@ -103,3 +103,102 @@ def test_weak_and_indefinite(k):
             assert np.abs(w[i] - w_o).max() < 1e-10 * max(1.0, np.abs(w_o).max())
         else:
             assert np.isnan(t[i]).all()
+
+
+def _failing_case(kind, k, rng):
+    y = rng.standard_normal((k, 5))
+    y -= y.mean(axis=0, keepdims=True)
+    dep, rloc, rinv = rng.standard_normal(5), np.ones(5), np.full(5, 0.5, np.float32)
+    if kind == "indefinite":                         # smallest eigenvalue -(k-1)/2
+        rinv[:] = -1.5 * (k - 1) / np.linalg.eigvalsh(y @ y.T).max()
+    elif kind == "nan":
+        y[rng.integers(k), 2] = np.nan
+    return y, rinv, dep, rloc
+
+
+# more failures than any list of them holds (256 per batch, 128 above k = 64)
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("k,n", [(20, 900), (64, 450), (100, 150)])
+def test_many_failures(k, n, noalloc):
+    """Good, indefinite and non-finite analyses in turn, after a call of the
+    same shape whose transforms are all finite: a non-finite analysis gives a
+    nonzero status and NaN outputs, an indefinite one NaN in trans (the square
+    root of a negative eigenvalue) and overline_w = M^-1 b, however many there
+    are.  Tolerance: a backward error of k eps |M| each for the tridiagonal form
+    and for QL, amplified by the condition of M."""
+    from dida_letkf import engine
+    if noalloc and k == 100:
+        n = 144                                      # what the fixed scratch holds
+    rng = np.random.default_rng(7 * k)
+    kinds = ["good" if i % 9 == 0 else "indefinite" if i % 2 else "nan" for i in range(n)]
+    assert sum(x != "good" for x in kinds) > (256 if k <= 64 else 120)
+    clean = [_failing_case("good", k, rng) for _ in kinds]
+    t, w, st = engine.letkf_core_batched(*[[c[i] for c in clean] for i in range(4)],
+                                         noalloc=noalloc)
+    assert (st == 0).all() and np.isfinite(t).all() and np.isfinite(w).all()
+    cases = [_failing_case(x, k, rng) for x in kinds]
+    t, w, st = engine.letkf_core_batched(*[[c[i] for c in cases] for i in range(4)],
+                                         noalloc=noalloc)
+    for i, (kind, (y, rinv, dep, _)) in enumerate(zip(kinds, cases)):
+        if kind == "nan":
+            assert st[i] != 0, i
+            assert np.isnan(t[i]).all() and np.isnan(w[i]).all(), i
+            continue
+        assert st[i] == 0, i
+        wy = y * rinv.astype(np.float64)
+        lam, v = np.linalg.eigh(wy @ y.T)
+        lam = lam + (k - 1)
+        tol = 2 * k * np.finfo(float).eps * np.abs(lam).max() / np.abs(lam).min()
+        w_o = v @ ((v.T @ (wy @ dep)) / lam)
+        assert np.abs(w[i] - w_o).max() <= max(tol, 1e-12) * max(1.0, np.abs(w_o).max()), i
+        if kind == "indefinite":
+            assert np.isnan(t[i]).all(), i
+        else:
+            t_o = (v * np.sqrt((k - 1) / lam)) @ v.T + w_o[:, None]
+            assert np.abs(t[i] - t_o).max() <= max(tol, 1e-12) * np.abs(t_o).max(), i
+
+
+@pytest.mark.parametrize("k,f32", [(20, False), (64, True), (100, False)])
+def test_many_failures_in_a_cycle(k, f32):
+    """Three cycles of one handle: good obs, obs whose Yb are NaN (every analysis
+    keeps its background and its transforms are NaN), obs of negative R^-1 (the
+    NaN of the square root reaches the state and is not counted as a failure,
+    as in the reference)."""
+    import copy
+
+    import torch
+    from dida_letkf import engine, synth
+    inst = synth.generate("c0", seed=k, k=k, nlat=16, nlon=30, n_obs=1500, local_dist=900.0)
+    cfg = inst.cfg
+    dt = torch.float32 if f32 else torch.float64
+    dev = torch.device("cuda:0")
+    xb = torch.from_numpy(np.ascontiguousarray(inst.xb)).to(dev).to(dt)
+    axb = torch.from_numpy(np.ascontiguousarray(inst.axb)).to(dev)
+    xa, axa = torch.zeros_like(xb), torch.zeros_like(axb)
+    h = cfg.halo
+    inner = (slice(h, h + cfg.nlon), slice(h, h + cfg.nlat))
+    with engine.LetkfEngine(cfg, keep_transforms=True) as eng:
+        eng.set_grid(inst.grid_lat, inst.grid_lon)
+        eng.set_stream(torch.cuda.current_stream().cuda_stream)
+        run = eng.analyze_device_f32 if f32 else eng.analyze_device
+
+        def cycle(obs):
+            eng.set_obs(obs)
+            rc = run(xb.data_ptr(), axb.data_ptr(), xa.data_ptr(), axa.data_ptr())
+            torch.cuda.synchronize()
+            return rc, eng.get_transforms()
+
+        rc, (t, w, nob) = cycle(inst.obs)
+        n = t.shape[0]
+        assert rc == 0 and np.isfinite(t).all() and n > 256 and (nob > 0).all()
+        bad = copy.deepcopy(inst.obs)
+        bad.yb[:, 1] = np.nan
+        rc, (t, w, _) = cycle(bad)
+        assert rc == n and eng.stats.n_flagged == n
+        assert np.isnan(t).all() and np.isnan(w).all()
+        assert torch.equal(xa[inner], xb[inner]) and torch.equal(axa[inner], axb[inner])
+        bad = copy.deepcopy(inst.obs)
+        bad.rinv[:] = -1e3 * np.abs(bad.rinv)
+        rc, (t, w, _) = cycle(bad)
+        assert rc == 0 and np.isnan(t).all() and np.isfinite(w).all()
+        assert torch.isnan(xa[inner]).all() and torch.isnan(axa[inner]).all()
