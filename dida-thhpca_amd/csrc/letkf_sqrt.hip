@@ -183,6 +183,7 @@ void k_vec(EigParams p) {
   __shared__ __align__(16) double sbuf[Lds::N];
   __shared__ double sb[KMAX], sw[KMAX];
   __shared__ double sred[4];
+  __shared__ int s_ok;                             // apart from sred: no barrier between them
   double* const sr = sbuf;                         // [KMAX][LDP]
   double* const sg = sr + KMAX * LDP;              // [KMAX][LDP], right after sr
   double* const sR = sg + KMAX * LDP;              // [TT][NP]
@@ -306,9 +307,9 @@ void k_vec(EigParams p) {
     N = kappa < 1e300 ? min((int)(1.86 * L + 0.8), 128) : NP;
     bool ok = chain(0);
     if constexpr (NW > 1) {
-      if (tid == 0) sred[0] = ok ? 1.0 : 0.0;
+      if (tid == 0) s_ok = ok;
       __syncthreads();
-      ok = sred[0] != 0.0;
+      ok = s_ok != 0;
       __syncthreads();
     }
     if (ok) break;

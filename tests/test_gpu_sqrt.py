@@ -202,3 +202,17 @@ def test_many_failures_in_a_cycle(k, f32):
         rc, (t, w, _) = cycle(bad)
         assert rc == 0 and np.isnan(t).all() and np.isfinite(w).all()
         assert torch.isnan(xa[inner]).all() and torch.isnan(axa[inner]).all()
+
+
+@pytest.mark.parametrize("k", [65, 97, 128])
+def test_four_wavefronts_same_bits(k):
+    """k > 64: the wavefronts of a matrix agree on its poles whatever runs beside
+    it.  Matrices of one to five groups of poles, in two orders: the same bits
+    for each."""
+    from dida_letkf import engine
+    cases = [_case(k, 40, 10.0 ** (i % 5), 50 * k + i) for i in range(60)]
+    args = [[c[i] for c in cases] for i in range(4)]
+    t, w, st = engine.letkf_core_batched(*args)
+    tr, wr, sr = engine.letkf_core_batched(*[a[::-1] for a in args])
+    assert (st == 0).all() and (sr == 0).all()
+    assert np.array_equal(t, tr[::-1]) and np.array_equal(w, wr[::-1])
