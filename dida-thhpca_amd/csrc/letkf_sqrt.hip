@@ -226,8 +226,9 @@ void k_vec(EigParams p) {
   // m: a lower bound of the spectrum.  0.9 (k-1)/rho holds for every A whose
   // negative rounding is small; it is checked beside the first poles' pivots
   // (lane NP tests that D - m has positive pivots), and where it fails the
-  // largest (0.9 / 2^t) (k-1)/rho that holds is taken.  None holding: D is not
-  // positive definite, and k_indef takes the matrix, or it is not finite.
+  // largest (0.9 / 2^t) (k-1)/rho that holds is taken, once.  None holding (or
+  // (k-1)/rho = 0, an infinite rho): D is not positive definite, or has no such
+  // bound, and k_indef takes the matrix, or it is not finite.
   double m = 0.9 * m0, L = 0.0, qn = 0.0;
   int N = 0;
   // pivots of the poles c0 .. c0 + NP - 1, one lane per pole (wavefront 0); a
@@ -300,7 +301,7 @@ void k_vec(EigParams p) {
     }
     return ok;
   };
-  for (;;) {
+  for (bool again = false;; again = true) {
     const double kappa = fmax(bound / m, 4.0);
     qn = 1.0 / (16.0 * kappa);
     L = -log(qn);
@@ -324,7 +325,7 @@ void k_vec(EigParams p) {
     }
     const unsigned long long bal = __builtin_amdgcn_ballot_w64(pos);
     const int f = bal ? __builtin_ctzll(bal) : 64;
-    if (f > 50 || !(bound < 1e290) || m < 0.9 * m0) {
+    if (again || !(m0 > 0.0) || f > 50 || !(bound < 1e290)) {
       // k_indef takes a finite matrix; nothing comes of one that is not
       bool fin = true;
       for (int i = lane; i < k; i += 64)

@@ -216,3 +216,30 @@ def test_four_wavefronts_same_bits(k):
     tr, wr, sr = engine.letkf_core_batched(*[a[::-1] for a in args])
     assert (st == 0).all() and (sr == 0).all()
     assert np.array_equal(t, tr[::-1]) and np.array_equal(w, wr[::-1])
+
+
+@pytest.mark.parametrize("rho", [np.inf, 1e308, 1e-300, 5e-324])
+@pytest.mark.parametrize("k,precision", [(20, 0), (64, 1), (100, 0)])
+def test_inflation_limits(k, precision, rho):
+    """(k-1)/rho = 0 (M = A, positive definite here: p > k rows that are not
+    centred), next to 0, huge and infinite (trans and overline_w 0): accepted
+    by the entry points, so every kernel ends and the result is the formula's.
+    Tolerance: k eps cond(A) for the tridiagonal form and the eigensolver
+    each, in FP32 the rounding of Yb and its sums, 1e-7, times that condition."""
+    from dida_letkf import engine
+    rng = np.random.default_rng(k)
+    p = 3 * k
+    y = rng.standard_normal((k, p))
+    rinv, dep, rloc = np.ones(p, np.float32), rng.standard_normal(p), np.ones(p)
+    t, w, st = engine.letkf_core_batched([y], [rinv], [dep], [rloc], inflation_factor=rho,
+                                         precision=precision)
+    assert st[0] == 0
+    lam, v = np.linalg.eigh(y @ y.T)
+    eps = np.finfo(float).eps if precision == 0 else 1e-7
+    tol = 2 * k * eps * lam.max() / lam.min()
+    with np.errstate(over="ignore", divide="ignore"):
+        lam = lam + np.float64(k - 1) / np.float64(rho)
+    w_o = v @ ((v.T @ (y @ dep)) / lam)
+    t_o = (v * np.sqrt((k - 1) / lam)) @ v.T + w_o[:, None]
+    assert np.abs(w[0] - w_o).max() <= tol * max(np.abs(w_o).max(), 1e-290)
+    assert np.abs(t[0] - t_o).max() <= tol * max(np.abs(t_o).max(), 1e-290)
