@@ -305,8 +305,10 @@ void k_vec(EigParams p) {
     const double kappa = fmax(bound / m, 4.0);
     qn = 1.0 / (16.0 * kappa);
     L = -log(qn);
-    N = kappa < 1e300 ? min((int)(1.86 * L + 0.8), 128) : NP;
-    bool ok = chain(0);
+    // sqrt_pole's terms stay finite up to 1e200 (862 poles)
+    const bool in_range = kappa <= 1e200;
+    N = in_range ? (int)(1.86 * L + 0.8) : 0;
+    bool ok = chain(0) && in_range;
     if constexpr (NW > 1) {
       if (tid == 0) s_ok = ok;
       __syncthreads();

@@ -243,3 +243,28 @@ def test_inflation_limits(k, precision, rho):
     t_o = (v * np.sqrt((k - 1) / lam)) @ v.T + w_o[:, None]
     assert np.abs(w[0] - w_o).max() <= tol * max(np.abs(w_o).max(), 1e-290)
     assert np.abs(t[0] - t_o).max() <= tol * max(np.abs(t_o).max(), 1e-290)
+
+
+@pytest.mark.parametrize("k", [4, 33, 70])
+@pytest.mark.parametrize("top", [1e13, 1e20, 1e60, 1e110])
+def test_wide_spectrum(k, top):
+    """Obs that each see one member: M is diagonal, its condition from 1e26 to
+    1e220, and trans and overline_w have closed forms.  Every term of the pole
+    sum is positive and each diagonal entry of the resolvents exact to a few ulp,
+    so the entries hold to 1e-13 of themselves (the sum over up to 862 poles
+    restated on the CPU: 5e-15)."""
+    from dida_letkf import engine
+    amp = np.logspace(0, np.log10(top), k - 1)
+    y = np.zeros((k, k - 1))
+    y[np.arange(k - 1), np.arange(k - 1)] = amp
+    dep = np.linspace(1.0, 2.0, k - 1)
+    one = np.ones(k - 1)
+    t, w, st = engine.letkf_core_batched([y], [one.astype(np.float32)], [dep], [one])
+    assert st[0] == 0
+    m = np.append(amp ** 2, 0.0) + (k - 1)
+    w_o = np.append(amp * dep, 0.0) / m
+    assert np.abs(w[0] / np.where(w_o > 0, w_o, 1.0) - (w_o > 0)).max() < 1e-13
+    d_o = np.sqrt((k - 1) / m)
+    diag = np.diagonal(t[0]) - w[0]
+    # taking overline_w off again costs an ulp of it
+    assert (np.abs(diag - d_o) <= 1e-13 * d_o + 4e-16 * w_o).all()
