@@ -2072,7 +2072,7 @@ static void launch_update(hipStream_t st, const EigParams& p, unsigned nb) {
 // smallest eigenvalue (reduced precision); trans and overline_w; update.  With
 // ql_first stages 1 and 2 are the QL recurrence and its rotations.
 template <int KMAX>
-static void launch_eig_stage_k(hipStream_t st, const EigParams& p, int stage) {
+static hipError_t launch_eig_stage_k(hipStream_t st, const EigParams& p, int stage) {
   const unsigned nb = (unsigned)p.n_an;
   const unsigned nq = (unsigned)((p.n_an + 63) / 64);
   if (stage == 0) {
@@ -2082,7 +2082,8 @@ static void launch_eig_stage_k(hipStream_t st, const EigParams& p, int stage) {
   } else if (stage == 3) {
     if (has_state(p)) launch_update<KMAX>(st, p, nb);
   } else if (!p.ql_first) {
-    (void)launch_sqrt(st, p, stage == 1);
+    const hipError_t e = launch_sqrt(st, p, stage == 1);
+    if (e != hipSuccess) return e;
     if (stage == 2)
       hipLaunchKernelGGL(k_indef<KMAX>, dim3((unsigned)std::min(p.n_an, 256LL)),
                          dim3(KMAX < 64 ? 64 : KMAX), 0, st, p);
@@ -2092,26 +2093,23 @@ static void launch_eig_stage_k(hipStream_t st, const EigParams& p, int stage) {
     if constexpr (KMAX == 128) hipLaunchKernelGGL(k_rot128, dim3(nb), dim3(256), 0, st, p);
     else hipLaunchKernelGGL(k_rot<KMAX>, dim3(nb), dim3(64), 0, st, p);
   }
+  return hipGetLastError();
 }
 
-static void launch_eig_stage(hipStream_t st, const EigParams& p, int stage) {
-  if (p.k <= 32) launch_eig_stage_k<32>(st, p, stage);
-  else if (p.k <= 64) launch_eig_stage_k<64>(st, p, stage);
-  else launch_eig_stage_k<128>(st, p, stage);
+static hipError_t launch_eig_stage(hipStream_t st, const EigParams& p, int stage) {
+  if (p.k <= 32) return launch_eig_stage_k<32>(st, p, stage);
+  if (p.k <= 64) return launch_eig_stage_k<64>(st, p, stage);
+  return launch_eig_stage_k<128>(st, p, stage);
 }
 
 hipError_t launch_eig(hipStream_t st, const EigParams& p, hipEvent_t* ev) {
   if (p.n_an <= 0) return hipSuccess;
   if (p.k > 128) return hipErrorInvalidValue;
   for (int stage = 0; stage < 4; ++stage) {
-    if (ev) {
-      const hipError_t e = hipEventRecord(ev[stage], st);
-      if (e != hipSuccess) return e;
-    }
-    launch_eig_stage(st, p, stage);
+    hipError_t e = ev ? hipEventRecord(ev[stage], st) : hipSuccess;
+    if (e == hipSuccess) e = launch_eig_stage(st, p, stage);
+    if (e != hipSuccess) return e;
   }
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
   return ev ? hipEventRecord(ev[4], st) : hipSuccess;
 }
 
