@@ -2588,7 +2588,8 @@ hipError_t launch_split(hipStream_t st, const SplitParams& p) {
 // by its cube count (:248-255).  The sums over m and c are one FP64 MFMA
 // chain per 16 members (16 elements x k by k x 16, over all covering cubes);
 // axb is left out of it and enters the mean only, so the members lose no
-// digits to its size.  A lane's operands of two consecutive steps are two
+// digits to its size (where it is not finite, dist_c(e) - mean_e dist_c is
+// NaN, and so are they).  A lane's operands of two consecutive steps are two
 // consecutive members of its element (A) and of its trans column (B), one
 // 16-byte load.
 // The bound is the load latency of trans (L2).  (A lane per member, each
@@ -2701,13 +2702,15 @@ void k_overlap_update(OverlapParams p, int ngrp,
     sum += dpp_d<0x140>(sum);
     const double mean = sum / k;
     if (v >= n) continue;
+    const double ab = p.axb[off + v];
+    const bool fin = __builtin_isfinite(ab);
     double* xac = p.xa + (off + v) * k;
 #pragma unroll
     for (int J = 0; J < TT; ++J) {
       const int e = 16 * J + i16;
-      if (e < k) xac[e] = (acc[J][r] - mean) / count;
+      if (e < k) xac[e] = fin ? (acc[J][r] - mean) / count : __builtin_nan("");
     }
-    if (i16 == 0) p.axa[off + v] = p.axb[off + v] + mean / count;
+    if (i16 == 0) p.axa[off + v] = ab + mean / count;
   }
 }
 

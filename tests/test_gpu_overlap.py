@@ -200,3 +200,37 @@ def test_overlap_update_widths(k, nz, cn, ov, halo):
     ref = orc.letkf_compute(inst, want_trans=True)
     got = _run(inst, precision=0, keep=True)
     assert rel(got["xa"], ref["xa"]) < TOL64 and rel(got["axa"], ref["axa"]) < TOL64
+
+
+@pytest.mark.parametrize("k,nz,cn,ov", [(20, 5, 4, 2), (100, 3, 3, 1)])
+def test_overlap_background_not_finite(k, nz, cn, ov):
+    """A NaN or Inf in the background mean or in a member spoils the members and
+    the mean of that state element, there and nowhere else, as in the oracle;
+    every other element is what it is without it."""
+    import copy
+
+    import orc
+    from dida_letkf import synth
+    inst = synth.generate("c2", seed=70 + k, k=k, nlat=9, nlon=14, nz=nz, n_obs=3000,
+                          local_dist=900.0)
+    inst.cfg.cube_n, inst.cfg.overlap = cn, ov
+    clean = _run(inst, precision=0, keep=True)
+    bad = copy.deepcopy(inst)
+    h, n = inst.cfg.halo, inst.axb.shape[2]
+    spots = [(h + 2, h + 3, 0, "axb", np.nan), (h + 5, h + 6, n - 1, "axb", np.inf),
+             (h + 9, h + 1, n // 2, "axb", -np.inf), (h + 11, h + 8, 1, "xb", np.nan)]
+    for jl, il, v, what, x in spots:
+        if what == "axb":
+            bad.axb[jl, il, v] = x
+        else:
+            bad.xb[jl, il, v, k // 2] = x
+    with np.errstate(all="ignore"):
+        ref = orc.letkf_compute(bad, want_trans=True)
+    got = _run(bad, precision=0, keep=True)
+    for name in ("xa", "axa"):
+        assert np.array_equal(np.isfinite(got[name]), np.isfinite(ref[name])), name
+        assert np.array_equal(np.isnan(got[name]), np.isnan(ref[name])), name
+        ok = np.isfinite(ref[name])
+        assert np.array_equal(got[name][ok], clean[name][ok]), name
+    for jl, il, v, _, _ in spots:
+        assert np.isnan(got["xa"][jl, il, v]).all() and not np.isfinite(got["axa"][jl, il, v])
