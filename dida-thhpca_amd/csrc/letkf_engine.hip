@@ -710,7 +710,7 @@ int dida_letkf_create(const dida_letkf_config* cfg, dida_letkf_handle** out) {
   h->bdeg_lat = 180.0 / h->nb_lat;
   h->bdeg_lon = 360.0 / h->nb_lon;
   h->max_batch = max_batch_columns(c);
-  h->tiled = h->nzc == 1 && h->kp <= 64 && c.products_kernel == 2;
+  h->tiled = !(c.vert_dist > 0.0) && h->kp <= 64 && c.products_kernel == 2;
   if (h->tiled) {
     // tiles never straddle batches, so results do not depend on the batching
     h->max_batch = std::max<long long>(kTile, (h->max_batch / kTile) * kTile);
@@ -1103,7 +1103,7 @@ static int prepare_call(dida_letkf_handle* h) {
     RC_TRY(h->row_site.ensure(sizeof(int) * rc));
   } else {
     RC_TRY(h->row_gc.ensure(sizeof(double) * (rc + kListPad)));
-    if (h->nzc == 1) RC_TRY(h->row_wd.ensure(sizeof(double) * (rc + kListPad)));
+    if (!(c.vert_dist > 0.0)) RC_TRY(h->row_wd.ensure(sizeof(double) * (rc + kListPad)));
   }
   if (c.keep_transforms || c.overlap > 0)
     RC_TRY(h->trans.ensure(sizeof(double) * h->n_an * c.k * c.k));
@@ -1257,8 +1257,9 @@ static int enqueue_call(dida_letkf_handle* h, const StateArgs& sa, bool timed, i
       sp.band_l = g.nlat_c;
     }
     // horizontal loop: weights precomputed by the fill pass (for the BF16
-    // products as the FP32 pair {sqrt(w), w dep})
-    sp.weights = h->nzc != 1 ? 0 : c.precision == DIDA_PREC_BF16X3 ? 2 : 1;
+    // products as the FP32 pair {sqrt(w), w dep}); with vertical localisation
+    // they depend on the level, also where a column is one chunk
+    sp.weights = c.vert_dist > 0.0 ? 0 : c.precision == DIDA_PREC_BF16X3 ? 2 : 1;
     sp.k = c.k;
     sp.rinv32 = h->rinv32.as<float>();
     sp.dep = h->o_dep.as<double>();
@@ -1309,7 +1310,7 @@ static int enqueue_call(dida_letkf_handle* h, const StateArgs& sa, bool timed, i
     pp.row_idx = h->row_idx.as<int>();
     pp.row_gc = h->row_gc.as<double>();
     pp.row_wd = h->row_wd.as<double>();
-    pp.pre_weighted = (!tiled && h->nzc == 1) ? 1 : 0;
+    pp.pre_weighted = !tiled && sp.weights != 0;
     pp.row_off = h->off.as<long long>();
     pp.row_cap = h->row_cap;
     pp.yb64 = h->o_yb64.as<double>();

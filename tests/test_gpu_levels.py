@@ -101,3 +101,27 @@ def test_level_products_support(k, nz, vert, n_obs):
                 xa2, axa2, rc2 = eng.letkf_compute(inst.xb, inst.axb)
                 assert np.isfinite(xa2).all() and np.isfinite(axa2).all()
                 assert rc2 > 0 and rc2 % nz == 0
+
+
+@pytest.mark.parametrize("k,nz,cube_nz,tile", [(20, 4, 4, 0), (33, 3, 32, 2), (100, 2, 2, 0),
+                                               (64, 5, 5, 2)])
+def test_level_products_one_chunk(k, nz, cube_nz, tile):
+    """A column that is one chunk of levels is localised in the vertical too (in
+    each precision, with the products kernel that tiles horizontal loops asked
+    for or not)."""
+    import orc
+    from dida_letkf import engine, synth
+    inst = synth.generate("c1", seed=k, k=k, nlat=6, nlon=11, nz=nz, n_obs=900, local_dist=700.0)
+    inst.cfg.vert_dist = 0.6
+    inst.cfg.cube_nz = cube_nz
+    ref = orc.letkf_compute(inst, want_trans=True)
+    full = ref["xa"] + ref["axa"][..., None]
+    inc = np.sqrt(np.mean((full - inst.xb - inst.axb[..., None]) ** 2))
+    for prec in (0, 1, 2):
+        got = engine.letkf_compute_nooverlap(inst, precision=prec, products_kernel=tile)
+        assert got["n_flagged"] == 0
+        got = got["xa"] + got["axa"][..., None]
+        if prec == 0:
+            assert np.abs(got - full).max() < 1e-10 * np.abs(full).max()
+        else:
+            assert np.sqrt(np.mean((got - full) ** 2)) < 1e-5 * inc
