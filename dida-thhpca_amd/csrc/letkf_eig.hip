@@ -387,16 +387,6 @@ __device__ __forceinline__ double block_sum(double v, double* red, int& slot) {
   }
 }
 
-__device__ __forceinline__ double block2_min(double v, double* red, int& slot) {
-  const double w = wave_min_full(v);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (lane == 0) red[2 * slot + wv] = w;
-  __syncthreads();
-  const double r = fmin(red[2 * slot], red[2 * slot + 1]);
-  slot ^= 1;
-  return uniform(r);
-}
-
 // ---------------------------------------------------------------------------
 // k_rot (ql_first): V (Q accumulation, logged rotations), overline_w and
 // trans = T + overline_w 1^T with LDS staged in small chunks, trans written
@@ -984,16 +974,6 @@ __device__ void copy_background_t(const EigParams& p, long long a) {
         }
       }
     }
-}
-
-__device__ void copy_background(const EigParams& p, long long a) {
-  if (p.epi) {
-    if (p.state_f32) copy_background_t<float, 1>(p, a);
-    else copy_background_t<double, 1>(p, a);
-  } else {
-    if (p.state_f32) copy_background_t<float, 0>(p, a);
-    else copy_background_t<double, 0>(p, a);
-  }
 }
 
 // k_update: xa(:, v) = trans^T xb(:, v) + axb(v), then re-centred, for the

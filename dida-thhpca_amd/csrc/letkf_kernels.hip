@@ -572,8 +572,8 @@ struct PairTable {
 // tiles [WS PPW, ...) of an analysis and, for WS = 0, b: the sums over rows
 // [r0, r1) (products_f64_rows) and their store (products_f64_store)
 template <int KP, int WS, int PPW, bool PW>
-__device__ __forceinline__ void products_f64_rows(const ProdParams& p, double vc, long long r0,
-                                                  long long r1, int lane, d4 (&acc)[PPW],
+__device__ __forceinline__ void products_f64_rows(const ProdParams& p, long long r0, long long r1,
+                                                  int lane, d4 (&acc)[PPW],
                                                   double (&bacc)[KP / 16]) {
   constexpr int T = KP / 16;
   using PT = PairTable<T>;
@@ -588,8 +588,7 @@ __device__ __forceinline__ void products_f64_rows(const ProdParams& p, double vc
   // G groups of 4 rows per step (lane q takes rows 4g + q), loaded one step
   // ahead of the MFMAs that use them; positions past the end of the row list
   // read its last row with zero weight (every load in bounds, no branch).
-  // More groups cost wavefronts per SIMD, which the per-row vertical weights
-  // of the k=32 level loop need more
+  // Two groups at k = 64: 14.8 -> 13.1 ms for 64,800 lists
   constexpr int G = KP == 64 ? 2 : 1;
   const int n = (int)(r1 - r0);
   auto load = [&](int rl, double* y, double& w, double& wd) {
@@ -600,7 +599,7 @@ __device__ __forceinline__ void products_f64_rows(const ProdParams& p, double vc
       wv = p.row_gc[r0 + rc];
       wdv = p.row_wd[r0 + rc];
     } else {
-      wv = row_weight(p, row, p.row_gc[r0 + rc], vc);
+      wv = (double)p.rinv32[row] * p.row_gc[r0 + rc];
       wdv = wv * p.dep[row];
     }
     const bool in = rl < n;
@@ -680,12 +679,11 @@ __device__ __forceinline__ void products_f64_store(const ProdParams& p, long lon
 }
 
 template <int KP, int WS, int PPW, bool PW>
-__device__ __forceinline__ void products_f64_wave(const ProdParams& p, long long a, int ah,
-                                                  double vc, long long r0, long long r1,
-                                                  int lane) {
+__device__ __forceinline__ void products_f64_wave(const ProdParams& p, long long a, long long r0,
+                                                  long long r1, int lane) {
   d4 acc[PPW];
   double bacc[KP / 16];
-  products_f64_rows<KP, WS, PPW, PW>(p, vc, r0, r1, lane, acc, bacc);
+  products_f64_rows<KP, WS, PPW, PW>(p, r0, r1, lane, acc, bacc);
   products_f64_store<KP, WS, PPW>(p, a, lane, acc, bacc);
 }
 
@@ -699,17 +697,16 @@ __global__ __launch_bounds__(256) void k_products_f64(ProdParams p) {
   const int wsub = wave % WPA;
   for_analyses<WPA, SCHED>(p, lane, [&](long long li) {
     const long long a = p.a0 + li;
-    const int ah = (int)(a / p.nzc), kc = (int)(a % p.nzc);
+    const int ah = (int)a;            // one analysis per column
     // row lists past the list buffer's capacity (the call then reruns with a
     // larger one) are cut at it, so no read leaves the buffer
     const long long r0 = min(p.row_off[ah - p.h0], p.row_cap);
     const long long r1 = min(p.row_off[ah - p.h0 + 1], p.row_cap);
-    const double vc = p.vertical ? chunk_vcoord(p, ah, kc) : 0.0;
-    if (wsub == 0) products_f64_wave<KP, 0, PPW, PW>(p, a, ah, vc, r0, r1, lane);
+    if (wsub == 0) products_f64_wave<KP, 0, PPW, PW>(p, a, r0, r1, lane);
     if constexpr (WPA > 1) {
-      if (wsub == 1) products_f64_wave<KP, 1, PPW, PW>(p, a, ah, vc, r0, r1, lane);
-      if (wsub == 2) products_f64_wave<KP, 2, PPW, PW>(p, a, ah, vc, r0, r1, lane);
-      if (wsub == 3) products_f64_wave<KP, 3, PPW, PW>(p, a, ah, vc, r0, r1, lane);
+      if (wsub == 1) products_f64_wave<KP, 1, PPW, PW>(p, a, r0, r1, lane);
+      if (wsub == 2) products_f64_wave<KP, 2, PPW, PW>(p, a, r0, r1, lane);
+      if (wsub == 3) products_f64_wave<KP, 3, PPW, PW>(p, a, r0, r1, lane);
     }
   });
 }
@@ -741,11 +738,11 @@ __global__ __launch_bounds__(512) void k_products_parts(ProdParams p) {
   const long long s0 = min(r0 + part * chunk, r1), s1 = min(s0 + chunk, r1);
   d4 acc[PPW];
   double bacc[T];
-  if (ws == 0) products_f64_rows<KP, 0, PPW, false>(p, 0.0, s0, s1, lane, acc, bacc);
+  if (ws == 0) products_f64_rows<KP, 0, PPW, false>(p, s0, s1, lane, acc, bacc);
   if constexpr (WPA > 1) {
-    if (ws == 1) products_f64_rows<KP, 1, PPW, false>(p, 0.0, s0, s1, lane, acc, bacc);
-    if (ws == 2) products_f64_rows<KP, 2, PPW, false>(p, 0.0, s0, s1, lane, acc, bacc);
-    if (ws == 3) products_f64_rows<KP, 3, PPW, false>(p, 0.0, s0, s1, lane, acc, bacc);
+    if (ws == 1) products_f64_rows<KP, 1, PPW, false>(p, s0, s1, lane, acc, bacc);
+    if (ws == 2) products_f64_rows<KP, 2, PPW, false>(p, s0, s1, lane, acc, bacc);
+    if (ws == 3) products_f64_rows<KP, 3, PPW, false>(p, s0, s1, lane, acc, bacc);
   }
 #pragma unroll
   for (int h = NR / 2; h >= 1; h /= 2) {
@@ -778,9 +775,8 @@ __global__ __launch_bounds__(512) void k_products_parts(ProdParams p) {
 }
 
 template <int KP, int WS, int PPW, bool PW>
-__device__ __forceinline__ void products_f32_wave(const ProdParams& p, long long a, int ah,
-                                                  double vc, long long r0, long long r1,
-                                                  int lane) {
+__device__ __forceinline__ void products_f32_wave(const ProdParams& p, long long a, long long r0,
+                                                  long long r1, int lane) {
   constexpr int T = KP / 16;
   using PT = PairTable<T>;
   constexpr int P0 = WS * PPW;
@@ -804,7 +800,7 @@ __device__ __forceinline__ void products_f32_wave(const ProdParams& p, long long
       w = p.row_gc[r0 + rc];
       wd = p.row_wd[r0 + rc];
     } else {
-      w = row_weight(p, row, p.row_gc[r0 + rc], vc);
+      w = (double)p.rinv32[row] * p.row_gc[r0 + rc];
       wd = w * p.dep[row];
     }
     const bool in = rl < n;
@@ -910,17 +906,16 @@ __global__ __launch_bounds__(256) void k_products_f32(ProdParams p) {
   const int wsub = wave % WPA;
   for_analyses<WPA, SCHED>(p, lane, [&](long long li) {
     const long long a = p.a0 + li;
-    const int ah = (int)(a / p.nzc), kc = (int)(a % p.nzc);
+    const int ah = (int)a;            // one analysis per column
     // row lists past the list buffer's capacity (the call then reruns with a
     // larger one) are cut at it, so no read leaves the buffer
     const long long r0 = min(p.row_off[ah - p.h0], p.row_cap);
     const long long r1 = min(p.row_off[ah - p.h0 + 1], p.row_cap);
-    const double vc = p.vertical ? chunk_vcoord(p, ah, kc) : 0.0;
-    if (wsub == 0) products_f32_wave<KP, 0, PPW, PW>(p, a, ah, vc, r0, r1, lane);
+    if (wsub == 0) products_f32_wave<KP, 0, PPW, PW>(p, a, r0, r1, lane);
     if constexpr (WPA > 1) {
-      if (wsub == 1) products_f32_wave<KP, 1, PPW, PW>(p, a, ah, vc, r0, r1, lane);
-      if (wsub == 2) products_f32_wave<KP, 2, PPW, PW>(p, a, ah, vc, r0, r1, lane);
-      if (wsub == 3) products_f32_wave<KP, 3, PPW, PW>(p, a, ah, vc, r0, r1, lane);
+      if (wsub == 1) products_f32_wave<KP, 1, PPW, PW>(p, a, r0, r1, lane);
+      if (wsub == 2) products_f32_wave<KP, 2, PPW, PW>(p, a, r0, r1, lane);
+      if (wsub == 3) products_f32_wave<KP, 3, PPW, PW>(p, a, r0, r1, lane);
     }
   });
 }
@@ -2466,12 +2461,19 @@ static hipError_t launch_products_sched(hipStream_t st, const ProdParams& p, int
   if (p.vertical && !w && precision == 1)
     return launch_prod(st, p, k_products_levels<KP, float, SCHED>, blocks, cl[1], WPA, capacity,
                        level_count<KP, float>());
+  // letkf_core's lists carry rho only; they come in plain order
+  if (!w && precision != 2) {
+    if constexpr (SCHED == 0)
+      return precision == 0
+                 ? launch_prod(st, p, k_products_f64<KP, 0, false>, blocks, c64[0], WPA, capacity)
+                 : launch_prod(st, p, k_products_f32<KP, 0, false>, blocks, c32[0], WPA, capacity);
+    else
+      return hipErrorInvalidValue;
+  }
   if (precision == 0)
-    return w ? launch_prod(st, p, k_products_f64<KP, SCHED, true>, blocks, c64[1], WPA, capacity)
-             : launch_prod(st, p, k_products_f64<KP, SCHED, false>, blocks, c64[0], WPA, capacity);
+    return launch_prod(st, p, k_products_f64<KP, SCHED, true>, blocks, c64[1], WPA, capacity);
   if (precision == 1)
-    return w ? launch_prod(st, p, k_products_f32<KP, SCHED, true>, blocks, c32[1], WPA, capacity)
-             : launch_prod(st, p, k_products_f32<KP, SCHED, false>, blocks, c32[0], WPA, capacity);
+    return launch_prod(st, p, k_products_f32<KP, SCHED, true>, blocks, c32[1], WPA, capacity);
   if (WPA == 1 && p.groups == 2)
     return w ? launch_prod(st, p, k_products_bf16<KP, 2, SCHED, true>, blocks, c16b[1], WPA,
                            capacity)
