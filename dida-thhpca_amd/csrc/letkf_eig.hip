@@ -750,8 +750,11 @@ void k_rot(EigParams p) {
 // status: thread 0 runs the QL recurrence a chase at a time, thread r applies
 // the chase's rotations to row r of Z in LDS.  Rare, so plain (a log of the
 // rotations, which k_ql_log keeps per matrix, would be four times the matrix);
-// a batch without such a matrix pays the launch and one read.
-// Runs before the update, which then takes every analysis in one pass.
+// a batch without such a matrix pays the launch and one read.  The bound is
+// thread 0's chain, one matrix per workgroup that fits the LDS: 4,050 of k = 20
+// 1.2 ms, of k = 64 4.7 ms, of k = 128 40 ms (the QL pass of a whole batch took
+// 0.4, 2.0 and 4.5).  Runs before the update, which then takes every analysis
+// in one pass.
 template <int KMAX>
 __global__ __launch_bounds__(KMAX < 64 ? 64 : KMAX) void k_indef(EigParams p) {
   if (*p.flag_n == 0) return;
@@ -2065,7 +2068,7 @@ static hipError_t launch_eig_stage_k(hipStream_t st, const EigParams& p, int sta
     const hipError_t e = launch_sqrt(st, p, stage == 1);
     if (e != hipSuccess) return e;
     if (stage == 2)
-      hipLaunchKernelGGL(k_indef<KMAX>, dim3((unsigned)std::min(p.n_an, 256LL)),
+      hipLaunchKernelGGL(k_indef<KMAX>, dim3((unsigned)std::min(p.n_an, KMAX < 128 ? 1024LL : 256LL)),
                          dim3(KMAX < 64 ? 64 : KMAX), 0, st, p);
   } else if (stage == 1) {
     hipLaunchKernelGGL(k_ql_log<KMAX>, dim3(nq), dim3(64), 0, st, p);
