@@ -31,6 +31,7 @@ sys.path.insert(0, os.path.join(ROOT, "oracle"))
 import numpy as np  # noqa: E402
 
 PEAK_FP64_TFLOPS = 78.6     # MI355X FP64 vector and FP64 matrix peak
+PEAK_FP32_TFLOPS = 157.3    # FP32 matrix
 PEAK_BF16_TFLOPS = 2500.0   # dense bf16 MFMA
 PEAK_HBM_GBS = 8000.0
 
@@ -51,27 +52,31 @@ def kernel_work(name, stats, cfg, n_an, mixed):
     products: the symmetric SYRK k(k+1) p plus Yb^T R^-1 d 2 k p flops per
               analysis (p local obs rows), on MFMA: the BF16 peak in the split
               mode (the three-term split's extra products are not counted),
-              FP64 otherwise;
+              else that of the mode's type.  Vertical loop: every row of a
+              column counts at every level, also where its weight is 0 and the
+              kernel leaves it out;
     apply:    T = V f V^T (2 k^3) and overline_w = Pa b (4 k^2) per analysis,
               FP64 MFMA; the reduction to tridiagonal form and the other work
               of the inverse square root are excluded from F and reported as
               a time share;
     update:   Xa = Xb trans, 2 k^2 m flops, HBM-bound: Xb read and Xa written
               (2 s_x k m bytes, s_x = 4 for the FP32 state of the mixed form,
-              8 for FP64) plus the means (16 m bytes) per analysis;
+              8 for FP64) plus the means (16 m bytes) per analysis of m state
+              vectors (n per column over its analyses);
     select, tridiag, ql: no F (index work, the tridiagonal form and its
               smallest eigenvalue).
     The FP64 vector and FP64 matrix peaks of MI355X are equal (78.6 TFLOP/s)."""
-    k, m = cfg.k, cfg.n
+    k, vectors = cfg.k, cfg.nlat * cfg.nlon * cfg.n
     if name == "products":
         p = stats["total_rows"]
         fl = k * (k + 1) * p + 2 * k * p
-        return fl, 0, (PEAK_BF16_TFLOPS if mixed == 2 else PEAK_FP64_TFLOPS), "mfma", "TFLOP/s"
+        peak = (PEAK_FP64_TFLOPS, PEAK_FP32_TFLOPS, PEAK_BF16_TFLOPS)[mixed]
+        return fl, 0, peak, "mfma", "TFLOP/s"
     if name == "apply":
         return n_an * (2 * k ** 3 + 4 * k ** 2), 0, PEAK_FP64_TFLOPS, "mfma", "TFLOP/s"
     if name == "update":
         sx = 4 if mixed else 8
-        return (n_an * 2 * k ** 2 * m, n_an * (2 * sx * k * m + 16 * m), PEAK_HBM_GBS / 1000.0,
+        return (vectors * 2 * k ** 2, vectors * (2 * sx * k + 16), PEAK_HBM_GBS / 1000.0,
                 "hbm", "TB/s")
     return 0, 0, PEAK_FP64_TFLOPS, "none", "TFLOP/s"
 
@@ -82,8 +87,8 @@ def cycle_work(stats, cfg, n_an, n_obs_rows, mixed):
     N_obs (s_y k + 40)."""
     k, m = cfg.k, cfg.n
     p = stats["total_rows"]
-    F = k * (k + 1) * p + 2 * k * p + n_an * (2 * k ** 3 + 4 * k ** 2 + 2 * k ** 2 * m)
     n_state = cfg.nlat * cfg.nlon * m
+    F = k * (k + 1) * p + 2 * k * p + n_an * (2 * k ** 3 + 4 * k ** 2) + 2 * k ** 2 * n_state
     sx = 4 if mixed else 8
     sy = 4 if mixed else 8
     B = 2 * sx * k * n_state + 16 * n_state + n_obs_rows * (sy * k + 40)
