@@ -32,7 +32,7 @@ __device__ __forceinline__ bool eig_slot(const EigParams& p, long long slot, lon
   return true;
 }
 
-// trans and overline_w of an analysis whose eigensolve failed on both passes
+// trans and overline_w of a failed analysis
 __device__ __forceinline__ void nan_transform(const EigParams& p, long long a) {
   const int k = p.k;
   const double nan = __longlong_as_double(0x7ff8000000000000LL);

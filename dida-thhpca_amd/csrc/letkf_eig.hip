@@ -5,8 +5,8 @@
 // The k x k matrices M = A + (k-1)/rho I of one batch are reduced to
 // tridiagonal form, and trans and overline_w follow from that form:
 //
-//   k_tridiag   one wavefront per matrix, lane r keeps row r of A in VGPRs;
-//               writes the reflectors, tau, and the tridiagonal (d, e)
+//   k_tridiag   one wavefront per matrix (k <= 32: two), lane r keeps row r of A
+//               in VGPRs; writes the reflectors, tau, and the tridiagonal (d, e)
 //   k_vec       trans and overline_w from the inverse square root of the
 //               tridiagonal form and its reflectors (letkf_sqrt.hip, with
 //               k_lmin before it for the reduced precisions' guard)
@@ -1715,8 +1715,9 @@ __device__ __forceinline__ void swap_rows(double&, double&) {}
 // lane quarters instead (v_permlane swaps) and keeps members 4 s + q.  LDS only
 // carries the wavefronts' shares of the means, one barrier a group.  (Staged through LDS
 // between two barriers a group, with no load in flight across them, and sums
-// by shuffles, 10.7 ms there; now about 6.4, cycle 63.1 ms; FP32 in the order of
-// the pieces 4.3 and 61.0 ms.)
+// by shuffles, 10.7 ms there; now 6.1, cycle 63.3 ms; FP32 in the order of
+// the pieces 4.3 and 61.0 ms.)  FP64 spills 32 registers, 72 with the epilogue:
+// its trans fills half of them.
 template <class TS, int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_update128(EigParams p) {

@@ -261,9 +261,10 @@ __global__ __launch_bounds__(1024) void k_call_summary(SummaryParams p) {
 // Scratch of the split eigensolver for one batch of analyses.
 struct EigScratch {
   DevBuf refl, tau, d, e, lam, rot, hdr, nchase;
-  // flags: [0] analyses the batch's first pass flagged, [1] the same summed
-  // over the batches of a call, [2 ..] their list; rr_*: the list pass's own
-  // scratch (its longer rotation log, chase headers, eigenvalues)
+  // flags: [0] analyses k_vec leaves to k_indef in the batch, [1] the analyses
+  // it flagged over the batches of a call; with ql_first also rot, hdr, nchase,
+  // [2 ..] the list of the list pass and rr_*, that pass's own scratch (its
+  // longer rotation log, chase headers, eigenvalues)
   DevBuf flags, rr_rot, rr_hdr, rr_nchase, rr_lam;
   std::vector<int> st_host;
 };
@@ -1996,7 +1997,7 @@ int core_run(hipStream_t st, CoreBufs& cb, EigScratch& es, int mode, int k, long
   pp.b = cb.b.as<double>();
   // One wavefront per analysis leaves most of the 1,024 SIMDs idle below that
   // many analyses, and each list is a chain; in parts, from two steps of rows
-  // a wavefront on (k = 64, 1,000 rows: 199 -> 47 us; 256 of k = 40: 92 -> 26)
+  // a wavefront on (k = 64, 1,000 rows: 199 -> 32 us; 256 of k = 40: 92 -> 19)
   if (precision == DIDA_PREC_FP64 && n_an <= 1024 && nr >= 32 * n_an)
     HIP_TRY(launch_products_parts(st, pp));
   else

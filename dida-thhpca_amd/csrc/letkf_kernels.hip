@@ -716,8 +716,9 @@ __global__ __launch_bounds__(256) void k_products_f64(ProdParams p) {
 // parts of four wavefronts), and the parts' sums meet in LDS pair by pair,
 // part h + i into part i.  A single list is a chain of row gathers: one
 // wavefront took 199 us for 1,000 rows of k = 64, and 92 us for 256 analyses
-// of up to 400 rows of k = 40; now 47 and 26 us (bound: the f64 MFMAs of one
-// CU, 17 us of them for the 1,000 rows).
+// of up to 400 rows of k = 40; now 32 and 19 us (bound: the f64 MFMAs of one
+// CU, 17 us of them for the 1,000 rows; 47 and 26 while the row loads still
+// held the branch of a vertical weight).
 template <int KP>
 __global__ __launch_bounds__(512) void k_products_parts(ProdParams p) {
   constexpr int T = KP / 16;
@@ -940,7 +941,7 @@ __global__ __launch_bounds__(256) void k_products_f32(ProdParams p) {
 // groups of 4 list positions (an MFMA step, a row per lane quarter), and every
 // row of the lists that flush: the same bits as with no row left out.
 // 360x180x32, k = 32, 3.2 G rows, FP32: 138 ms with weights beside the MFMAs,
-// 55 ms with blocks of 64 unfiltered rows, about 40 ms now (cycle 91 ms; row by
+// 55 ms with blocks of 64 unfiltered rows, 42 ms now (cycle 91 ms; row by
 // row 22 and 72).
 template <class REAL> struct LevelReal;
 template <> struct LevelReal<double> {
@@ -963,8 +964,11 @@ template <> struct LevelReal<float> {
 };
 
 // levels per visit: the accumulators of LV levels (tiles x 4 registers, 8 for
-// FP64) beside the loads in flight against wavefronts per SIMD (k = 32 FP32:
-// 2 levels 55 ms, 4 64 ms, 8 80 ms)
+// FP64) beside the loads in flight against wavefronts per SIMD (k = 32 FP32,
+// unfiltered rows: 2 levels 55 ms, 4 64 ms, 8 80 ms).  k = 64 and 128 hold one
+// or two wavefronts a SIMD for it, against three of the kernel with one level
+// and its weights beside the MFMAs: 120x60x16 FP32 5.6 -> 2.9 and 23.5 -> 17.2
+// ms, FP64 (one level) 9.4 -> 3.0 and 40.0 -> 12.8
 template <int KP, class REAL>
 constexpr int level_count() {
   return KP == 32 || sizeof(REAL) == 4 ? 2 : 1;

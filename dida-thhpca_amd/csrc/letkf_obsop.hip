@@ -254,7 +254,7 @@ static hipError_t launch_obs_operator_s(hipStream_t st, const ObsOpParams& p) {
 hipError_t launch_obs_operator(hipStream_t st, const ObsOpParams& p) {
   if (p.n_sites <= 0) return hipSuccess;
   // four sites a wavefront from the count on whose wavefronts still fill the
-  // chip (256 CUs of 32): 201k sites 789 -> 375..448 us; below it a site's own
+  // chip (256 CUs of 32): 201k sites 789 -> 448 us; below it a site's own
   // chain is what a call waits for (40 of them: 23 -> 20 us a call)
   return p.n_sites >= 4 * 8192 ? launch_obs_operator_s<4>(st, p) : launch_obs_operator_s<1>(st, p);
 }

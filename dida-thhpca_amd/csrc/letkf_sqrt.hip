@@ -29,9 +29,9 @@
 //
 // It replaces the QL recurrence and the product of its rotations (k_indef keeps
 // them for M not positive definite), ~4,500 dependent Givens steps per matrix at k = 64
-// and 6 k flops for each.  64,800 matrices: k = 64, 3.95 + 7.25 -> 0.21
-// (k_lmin) + 2.40 ms; k = 128, 50 + 80 -> 0.5 + 20 ms; and a single matrix of
-// k = 64 takes 60 us here against 1.3 ms.  Bound: the wavefront's own chain
+// and 6 k flops for each.  64,800 matrices: k = 64, 3.95 + 7.25 -> 0.22
+// (k_lmin) + 2.5 ms; k = 128, 50 + 80 -> 0.43 + 20 ms; and a single matrix of
+// k = 64 takes 50 us here against 1.3 ms.  Bound: the wavefront's own chain
 // (per matrix of k = 64 some 150k cycles with two wavefronts on a SIMD, of
 // which 47k are MFMA issue; the pivots 25k, W 20k, the last stores 15k).
 #include "letkf_device.h"
@@ -171,8 +171,8 @@ struct SqrtLds {
 };
 
 // k <= 32: three wavefronts per SIMD hide more of each one's chain than the
-// spills they cost (228 B a lane): 2,073,600 matrices 28 -> 24 ms, four
-// wavefronts 31 ms.  k > 32 spills at two already.
+// spills they cost (200 B a lane): 2,073,600 matrices 28 -> 25 ms, four
+// wavefronts 31 ms.  k > 32 spills at two already (k = 64: 196 B, k = 128: 340).
 template <int KMAX, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(KMAX == 32 ? 3 : 2)))
 void k_vec(EigParams p) {

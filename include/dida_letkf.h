@@ -112,8 +112,9 @@ typedef struct dida_letkf_stats {
     long long n_analyses;   /* local analyses (k x k transform solves) */
     long long total_rows;   /* sum of local obs rows over analyses */
     int max_rows;           /* largest local obs count */
-    int n_flagged;          /* analyses whose eigensolve failed on both passes (their
-                               state keeps the background: xa = xb, axa = axb) */
+    int n_flagged;          /* analyses whose eigensolve failed or whose obs terms are not
+                               finite (their state keeps the background: xa = xb,
+                               axa = axb) */
     int rows_over_10000;    /* analyses the reference's MAX_OBS would truncate */
     double ms_select;       /* device time, local obs selection */
     double ms_products;     /* device time, obs-space products */
